@@ -105,8 +105,9 @@ struct mi355nufft_plan {
     hipStream_t stream = nullptr;
 
     void* d_tab[3] = {nullptr, nullptr, nullptr};  // full tables (J*L+1 entries)
-    void* d_tw[3] = {nullptr, nullptr, nullptr};   // FFT twiddles exp(-2 pi i m / K_d), complex T
-    int fft_fused_ok = 0;  // every K_d a power of two in [kFftMinK, kFftMaxK]
+    void* d_tw[3] = {nullptr, nullptr, nullptr};   // FFT twiddles, complex T, one section per pass (FftAxis)
+    FftAxis fft_ax[3] = {};
+    int fft_fused_ok = 0;  // every K_d has fused passes (fused_fft_sizes_ok)
     int fft_method = 0;    // 0 auto (fused pruned FFT when possible), 1 rocFFT
     // set while mi355nufft_forward / _adjoint run with phase_before (and the
     // forward's ortho scale) applied by the fused FFT passes instead of the
@@ -366,6 +367,7 @@ struct FftDev {
     int ndim;
     int64_t N[3], K[3], nk;
     void* const* tw;
+    const FftAxis* ax;
     const double* const* sn;
     hipStream_t stream;
 };
@@ -379,15 +381,22 @@ inline FftDev fft_dev(const mi355nufft_plan* p) {
     }
     f.nk = p->nk;
     f.tw = p->d_tw;
+    f.ax = p->fft_ax;
     f.sn = p->d_sn;
     f.stream = p->stream;
     return f;
 }
 
 
+// Passes, twiddle sections and threads per line of an axis of length K:
+// power-of-two lengths in [kFftMinK, kFftMaxK] and lengths whose prime
+// factors are 2, 3, 5 and 7; false for any other (fft.hip).
+bool fft_axis_init(int64_t K, FftAxis* ax);
+inline bool fft_pow2(int64_t k) { return (k & (k - 1)) == 0; }
+
 // Options of one pass: rezero (adjoint: leave the grid it reads all zero),
 // mult (adjoint: multiply the loaded spectrum by this grid-shaped array),
-// pb (column pass of an ndim >= 2 power-of-two grid: 1 multiplies the
+// pb (column pass of an ndim >= 2 grid: 1 multiplies the
 // output by phase_before and divides by scale_ortho if ortho, 2 multiplies
 // the input by conj(phase_before); pbc null means a zero phase).
 struct FftPassOpts {
