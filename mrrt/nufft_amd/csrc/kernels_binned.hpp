@@ -684,6 +684,7 @@ __device__ __forceinline__ float block_sum(float v, float* red) {
 
 // MULTI: repetitions (coils) are processed a.rc at a time: a.rc tiles are
 // staged, and each point's coefficients are computed once for all of them.
+// Workgroup (x, y) takes every gridDim.y-th pass over the repetitions.
 // FUSED: the tap sums use fused multiply-adds.
 template <typename T, int NDIM, bool CK, int JMAX, bool FIXED, bool MULTI, bool FUSED = false>
 __global__ __launch_bounds__(256) void interp_tiled_kernel(TiledArgs<T, CK> a) {
@@ -699,7 +700,7 @@ __global__ __launch_bounds__(256) void interp_tiled_kernel(TiledArgs<T, CK> a) {
         Sub s;
         load_sub(bg, a.bs, NDIM, sid, s);
         if constexpr (!MULTI) {
-            for (int r = 0; r < ia.nreps; ++r) {
+            for (int r = blockIdx.y; r < ia.nreps; r += gridDim.y) {
                 stage_tile<T, NDIM, CK>(a, s, ax, ia.grid + ((int64_t)s.frame * ia.nreps + r) * ia.kstride, tiles);
                 __syncthreads();
                 if constexpr (NDIM >= 2) {
@@ -748,7 +749,7 @@ __global__ __launch_bounds__(256) void interp_tiled_kernel(TiledArgs<T, CK> a) {
             }
             continue;
         }
-        for (int r0 = 0; r0 < ia.nreps; r0 += a.rc) {
+        for (int r0 = blockIdx.y * a.rc; r0 < ia.nreps; r0 += gridDim.y * a.rc) {
             const int rc = min(a.rc, ia.nreps - r0);
             for (int rr = 0; rr < rc; ++rr)
                 stage_tile<T, NDIM, CK>(a, s, ax, ia.grid + ((int64_t)s.frame * ia.nreps + r0 + rr) * ia.kstride,
@@ -845,7 +846,7 @@ __global__ __launch_bounds__(256) void spread_tiled_kernel(TiledArgs<T, CK> a) {
         const int i1 = ic + blockDim.x;
         // RC repetitions per pass, each with its own tile: one barrier round
         // and one coefficient computation per point serve all of them
-        for (int r0 = 0; r0 < ia.nreps; r0 += RC) {
+        for (int r0 = blockIdx.y * RC; r0 < ia.nreps; r0 += gridDim.y * RC) {
             const int rc = min(RC, ia.nreps - r0);  // uniform over the workgroup
             for (int e = tid; e < 2 * rc * bg.tile; e += blockDim.x) tiles[e] = 0;
             int sh[RC];     // FXP: tap values of repetition r0 + k are scaled by 2^sh[k]
