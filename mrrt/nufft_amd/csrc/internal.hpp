@@ -19,6 +19,7 @@
 #include "kernels_grid.hpp"
 #include "kernels_interp.hpp"
 #include "kernels_binned.hpp"
+#include "kernels_owner.hpp"
 #include "kernels_fft.hpp"
 #include "kernels_sparse.hpp"
 
@@ -129,6 +130,10 @@ struct mi355nufft_plan {
     // zero again and the next scatter needs no separate clear
     void* d_agrid = nullptr;
     size_t agrid_bytes = 0;
+    // grid of adjoints whose scatter writes every cell (use_owner): neither
+    // cleared before nor left zero after
+    void* d_ogrid = nullptr;
+    size_t ogrid_bytes = 0;
     int agrid_zero = 0;  // d_agrid holds zeros (host-side state, stream order)
 
     // binning (tiled kernels)
@@ -159,7 +164,7 @@ struct mi355nufft_plan {
     int binned = 0;           // bin state valid for the current points
     int* d_bin_i = nullptr;   // one allocation: bin_of, rank, perm (3*M_cap)
     int* d_bin_b = nullptr;   // counts, bin_start, bin_sub, bank-key counts ((3 + kBanks) * nbins_cap)
-    int* d_sub = nullptr;     // sub_bin, sub_start, sub_end (3*sub_cap) + n_sub
+    int* d_sub = nullptr;     // sub_bin, sub_start, sub_end (3*sub_cap) + n_sub, max_count
     void* d_tms = nullptr;    // tm in sorted order (ndim * M_cap real)
     void* d_phs = nullptr;    // per-sample phase in sorted order (M_cap complex)
     int64_t sorted_cap = 0;
@@ -242,6 +247,7 @@ inline BinState bin_state(const mi355nufft_plan* p) {
     bs.sub_start = p->d_sub + sc;
     bs.sub_end = p->d_sub + 2 * sc;
     bs.n_sub = p->d_sub + 3 * sc;
+    bs.max_count = bs.n_sub + 1;
     bs.frame_off = p->nframes > 1 ? p->d_frame_off : nullptr;
     bs.nframes = p->nframes;
     return bs;
@@ -301,6 +307,38 @@ inline int fixed_j(int ndim, const int32_t* Jd) {
     return Jd[0] == 6 ? 6 : 0;
 }
 
+
+// Whether the scatter of nreps repetitions runs spread_owner_kernel: 2-D
+// fixed-point tiles whose geometry it takes (the bins that reach one owned
+// tile fit its list, the periodic range of a tile does not meet itself) with
+// grids that together are too large for the caches and at most one point per
+// two cells.  Whole adjoints, owner / atomic: 24 frames x 32 coils of Kd
+// 512^2 (1.6 GB) 2.50 / 4.96 ms, 4 x 32 (256 MB) 519 / 831 us, 2 x 32
+// (128 MB) 274 / 355 us, 2 x 8 (32 MB) 172 / 113 us; 128 coils of one
+// trajectory (256 MB) with 0.25 random points per cell 600 / 1068 us, 0.5
+// 990 / 1162, 0.79 1632 / 1295.
+constexpr size_t kOwnerMinBytes = (size_t)128 << 20;
+constexpr int kOwnerMinReps = 4;
+inline int owner_stride(const mi355nufft_plan* p) {
+    const int need = kOwnerB + 2 * (p->J[0] - 1);
+    return need + (((p->bg.T[0] - need) % 32 + 32) % 32);
+}
+inline size_t owner_plane_bytes(const mi355nufft_plan* p) {
+    return (size_t)owner_stride(p) * (kOwnerB + 2 * (p->J[1] - 1)) * 2 * sizeof(int);
+}
+inline bool use_owner(const mi355nufft_plan* p, int32_t nreps) {
+    if (p->ndim != 2 || !use_tiled(p) || !use_fxp(p) || (p->method != 0 && p->method != 2)) return false;
+    const int64_t cells = p->nframes * p->nk;
+    if (nreps < kOwnerMinReps || 2 * p->M > cells || (size_t)cells * nreps * p->cx_size() < kOwnerMinBytes)
+        return false;
+    int segs = 1;
+    for (int d = 0; d < 2; ++d) {
+        const int J = p->J[d], B = p->bg.B[d];
+        if (J > kOwnerMaxJ || p->K[d] < kOwnerB + 2 * (J - 1)) return false;
+        segs *= (kOwnerB + J - 2) / B + 3;  // the range, cut by bins and by the wrap
+    }
+    return segs <= kOwnerSegs && p->bg_threads == 256 && 2 * owner_plane_bytes(p) <= p->lds_limit / 2;
+}
 
 // The bin sort of the plan's points (p->d_tm, p->M, p->bg) into its binning
 // storage, in six launches: clear the (bin, bank key) counters, count, sum

@@ -45,6 +45,7 @@ struct BinState {
     int* sub_start;  // (max_sub) first sorted position of each subproblem
     int* sub_end;    // (max_sub) one past its last sorted position
     int* n_sub;      // (1) number of subproblems
+    int* max_count;  // (1) points of the fullest bin
     int* bin_sub;    // (nbins) first subproblem of each bin
     int* bkt;        // (nbins * kBanks) points per (bin, bank key)
     const int64_t* frame_off;  // (nframes + 1) first point of each frame, or null
@@ -134,9 +135,10 @@ static __global__ __launch_bounds__(1024) void bin_scan_kernel(BinState bs, int 
     const int chunk = (nbins + 1023) / 1024;
     const int b0 = tid * chunk;
     const int b1 = min(nbins, b0 + chunk);
-    int pts = 0, subs = 0;
+    int pts = 0, subs = 0, top = 0;
     for (int b = b0; b < b1; ++b) {
         const int c = bs.counts[b];
+        top = max(top, c);
         pts += c;
         subs += (c + P - 1) / P;
     }
@@ -171,6 +173,13 @@ static __global__ __launch_bounds__(1024) void bin_scan_kernel(BinState bs, int 
         run_s += ns;
     }
     if (tid == 1023) bs.n_sub[0] = min(s_sub[1023], max_sub);
+    __syncthreads();
+    s_pts[tid] = top;
+    for (int off = 512; off > 0; off >>= 1) {
+        __syncthreads();
+        if (tid < off) s_pts[tid] = max(s_pts[tid], s_pts[tid + off]);
+    }
+    if (tid == 0) bs.max_count[0] = s_pts[0];
 }
 
 // Sorted position of point m.  Its place in the bin's (rank, key) order is
@@ -251,6 +260,7 @@ struct TiledArgs {
     int own_ok;             // scatter: every K_d is a multiple of B_d (see spread_tiled_kernel)
     float cmax;             // scatter: > 0 accumulates in fixed point; bound of |coefficient product|
     int exact;              // gather: 1 keeps the reference's roundings (no fused multiply-add)
+    int heavy;              // scatter after spread_owner_kernel: only bins of more points (0: all)
     unsigned long long* flush_count;  // scatter: non-null adds the flush's global atomic lane operations
     int flush_slots;                  // power of two: workgroup b adds to flush_count[b % flush_slots]
 };
@@ -829,7 +839,9 @@ __global__ __launch_bounds__(256) void spread_tiled_kernel(TiledArgs<T, CK> a) {
     const int tid = threadIdx.x;
     const int n_sub = a.bs.n_sub[0];
     unsigned natom = 0;  // global atomic lane operations of this thread's flushes
+    if (a.heavy > 0 && a.bs.max_count[0] <= a.heavy) return;
     for (int sid = blockIdx.x; sid < n_sub; sid += gridDim.x) {
+        if (a.heavy > 0 && a.bs.counts[a.bs.sub_bin[sid]] <= a.heavy) continue;
         Sub s;
         load_sub(bg, a.bs, NDIM, sid, s);
         // REPS: this thread's point (sorted position ic), coefficients cached

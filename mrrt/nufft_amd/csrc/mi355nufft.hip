@@ -194,20 +194,25 @@ bool stream_capturing(const mi355nufft_plan* p) {
     return cs != hipStreamCaptureStatusNone;
 }
 
+// plan-owned scratch of nimg grids, grown on demand
+int grow_grid(mi355nufft_plan* p, int32_t nimg, void** buf, size_t* bytes) {
+    const size_t need = (size_t)nimg * (size_t)p->nk * p->cx_size();
+    if (need > *bytes) {
+        if (*buf) {
+            HIP_TRY(hipStreamSynchronize(p->stream));
+            HIP_TRY(hipFree(*buf));
+            *buf = nullptr;
+            *bytes = 0;
+        }
+        if (hipMalloc(buf, need) != hipSuccess) return fail(MI355NUFFT_ENOMEM, "grid scratch of %zu bytes", need);
+        *bytes = need;
+    }
+    return MI355NUFFT_OK;
+}
+
 int get_grid(mi355nufft_plan* p, int32_t nreps, void** grid) {
     if (*grid) return MI355NUFFT_OK;
-    const size_t need = (size_t)nreps * (size_t)p->nk * p->cx_size();
-    if (need > p->grid_bytes) {
-        if (p->d_grid) {
-            HIP_TRY(hipStreamSynchronize(p->stream));
-            HIP_TRY(hipFree(p->d_grid));
-            p->d_grid = nullptr;
-            p->grid_bytes = 0;
-        }
-        if (hipMalloc(&p->d_grid, need) != hipSuccess)
-            return fail(MI355NUFFT_ENOMEM, "grid scratch of %zu bytes", need);
-        p->grid_bytes = need;
-    }
+    RET_IF(grow_grid(p, nreps, &p->d_grid, &p->grid_bytes));
     *grid = p->d_grid;
     return MI355NUFFT_OK;
 }
@@ -696,7 +701,7 @@ template <typename T>
 int spread_impl(mi355nufft_plan* p, const void* y, void* grid, int32_t nreps, bool grid_is_zero = false) {
     if (p->sp.on) return sparse_spread<T>(p, y, grid, nreps, false);  // writes every grid point
     if (use_tiled(p) && use_two_phase(p, nreps)) return spread_two_phase<T>(p, y, grid, nreps);
-    if (!grid_is_zero) RET_IF(zero_grid<T>(grid, (int64_t)p->nframes * nreps * p->nk, p->stream));
+    if (!grid_is_zero && !use_owner(p, nreps)) RET_IF(zero_grid<T>(grid, (int64_t)p->nframes * nreps * p->nk, p->stream));
     if (use_tiled(p)) return run_tiled_any<T>(p, true, y, nullptr, nullptr, grid, nreps);
     if (p->nframes > 1) return fail(MI355NUFFT_ESTATE, "frames need the tiled kernels");
     int32_t J[3] = {p->J[0], p->J[1], p->J[2]};
@@ -817,7 +822,7 @@ int grow(mi355nufft_plan* p, Tp** buf, int64_t& cap, int64_t need, int64_t per) 
         *buf = nullptr;
         cap = 0;
     }
-    if (hipMalloc((void**)buf, (size_t)(need * per + 1) * sizeof(Tp)) != hipSuccess)
+    if (hipMalloc((void**)buf, (size_t)(need * per + 2) * sizeof(Tp)) != hipSuccess)
         return fail(MI355NUFFT_ENOMEM, "binning storage (%lld entries)", (long long)(need * per));
     cap = need;
     return MI355NUFFT_OK;
@@ -1079,7 +1084,7 @@ RawLayout raw_layout(int64_t M, int ndim, size_t rs, int64_t nbins, int64_t max_
     L.bin_b = o;
     o = up(o + (size_t)(kBanks + 3) * (size_t)nbins * sizeof(int));
     L.sub = o;
-    o = up(o + (size_t)(3 * max_sub + 1) * sizeof(int));
+    o = up(o + (size_t)(3 * max_sub + 2) * sizeof(int));
     L.tms = o;
     o = up(o + (size_t)ndim * (size_t)M * rs);
     L.total = o;
@@ -1421,6 +1426,7 @@ int mi355nufft_plan_destroy(mi355nufft_plan* p) {
     if (p->d_phase) (void)hipFree(p->d_phase);
     if (p->d_grid) (void)hipFree(p->d_grid);
     if (p->d_agrid) (void)hipFree(p->d_agrid);
+    if (p->d_ogrid) (void)hipFree(p->d_ogrid);
     if (p->fft_work) (void)hipFree(p->fft_work);
     if (p->d_bin_i) (void)hipFree(p->d_bin_i);
     if (p->d_bin_b) (void)hipFree(p->d_bin_b);
@@ -1910,6 +1916,11 @@ int mi355nufft_adjoint(mi355nufft_plan* p, const void* y, void* x, const int64_t
     // phase: the first inverse FFT pass applies conj(phase_before) instead of
     // the scatter's flush
     const int phase = fft_phase_adjoint(p, nreps) ? 2 : 0;
+    if (!grid && !p->sp.on && use_owner(p, nreps)) {
+        // every cell is written: a grid of its own, which no pass has to clear
+        RET_IF(grow_grid(p, nimg, &p->d_ogrid, &p->ogrid_bytes));
+        grid = p->d_ogrid;
+    }
     if (grid) {
         if (!phase) {
             RET_IF(mi355nufft_spread(p, y, grid, nreps));
