@@ -30,7 +30,7 @@ void launch_tiled(bool adjoint, const TiledArgs<T, CK>& a, unsigned nsub, unsign
                                  : spread_tiled_kernel<T, NDIM, CK, JMAX, FIXED, true, false>;
     auto interp = a.rc > 1 ? interp_tiled_kernel<T, NDIM, CK, JMAX, FIXED, true>
                            : interp_tiled_kernel<T, NDIM, CK, JMAX, FIXED, false>;
-    if constexpr (FIXED)  // fused tap sums for the J = 6 kernels unless the reference's roundings are asked for
+    if constexpr (FIXED)  // fused tap sums unless the reference's roundings are asked for
         if (!a.exact)
             interp = a.rc > 1 ? interp_tiled_kernel<T, NDIM, CK, JMAX, FIXED, true, true>
                               : interp_tiled_kernel<T, NDIM, CK, JMAX, FIXED, false, true>;
@@ -86,6 +86,8 @@ int launch_owner(mi355nufft_plan* p, const TiledArgs<float, CK>& a, hipEvent_t e
 template <bool CK>
 int run_owner(mi355nufft_plan* p, const TiledArgs<float, CK>& a, hipEvent_t ev0) {
     const int j = p->J[0] == p->J[1] ? p->J[0] : 0;
+    if (j == 4) return launch_owner<CK, 4, true>(p, a, ev0);
+    if (j == 5) return launch_owner<CK, 5, true>(p, a, ev0);
     if (j == 6) return launch_owner<CK, 6, true>(p, a, ev0);
     if (p->J[0] <= 4 && p->J[1] <= 4) return launch_owner<CK, 4, false>(p, a, ev0);
     return launch_owner<CK, 8, false>(p, a, ev0);
@@ -152,6 +154,8 @@ int run_tiled(mi355nufft_plan* p, bool adjoint, const void* samples_in, void* sa
         LAUNCH_CHECK();                                                        \
         return MI355NUFFT_OK;                                                  \
     }
+    MI355_FCASE(1, 4) MI355_FCASE(2, 4) MI355_FCASE(3, 4)
+    MI355_FCASE(1, 5) MI355_FCASE(2, 5) MI355_FCASE(3, 5)
     MI355_FCASE(1, 6) MI355_FCASE(2, 6) MI355_FCASE(3, 6)
 #undef MI355_FCASE
 #define MI355_TCASE(ND, JM)                                                  \
@@ -218,6 +222,8 @@ int run_grad(mi355nufft_plan* p, const void* grid, const void* w, void* grad, in
         LAUNCH_CHECK();                                                \
         return MI355NUFFT_OK;                                          \
     }
+    MI355_GFCASE(1, 4) MI355_GFCASE(2, 4) MI355_GFCASE(3, 4)
+    MI355_GFCASE(1, 5) MI355_GFCASE(2, 5) MI355_GFCASE(3, 5)
     MI355_GFCASE(1, 6) MI355_GFCASE(2, 6) MI355_GFCASE(3, 6)
 #undef MI355_GFCASE
 #define MI355_GCASE(ND, JM)                                            \
