@@ -314,12 +314,15 @@ inline int fixed_j(int ndim, const int32_t* Jd) {
 // fixed-point tiles whose geometry it takes (the bins that reach one owned
 // tile fit its list, the periodic range of a tile does not meet itself) with
 // grids that together are too large for the caches and at most one point per
-// two cells.  Whole adjoints, owner / atomic: 24 frames x 32 coils of Kd
-// 512^2 (1.6 GB) 2.50 / 4.96 ms, 4 x 32 (256 MB) 519 / 831 us, 2 x 32
-// (128 MB) 274 / 355 us, 2 x 8 (32 MB) 172 / 113 us; 128 coils of one
-// trajectory (256 MB) with 0.25 random points per cell 600 / 1068 us, 0.5
-// 990 / 1162, 0.79 1632 / 1295.
+// two cells; the atomic kernel keeps up longer with bins larger than 16x16.
+// Whole adjoints, owner / atomic: 32x32 bins, 24 frames x 32 coils of Kd
+// 512^2 (1.6 GB) 2.31 / 3.12 ms, 12 x 16 (384 MB) 694 / 753 us, 24 x 6 (288
+// MB) 578 / 581, 8 x 16 (256 MB) 531 / 509; 16x16 bins, 128 coils of one
+// trajectory (256 MB) with 0.25 random points per cell 596 / 1068 us, 0.5
+// 993 / 1163, 0.79 1632 / 1295, 64 coils (128 MB) with 0.25 286 / 512, 0.5
+// 440 / 547, 2 x 8 coils (32 MB) 172 / 113.
 constexpr size_t kOwnerMinBytes = (size_t)128 << 20;
+constexpr size_t kOwnerMinBytesLarge = (size_t)320 << 20;
 constexpr int kOwnerMinReps = 4;
 inline int owner_stride(const mi355nufft_plan* p) {
     const int need = kOwnerB + 2 * (p->J[0] - 1);
@@ -331,7 +334,8 @@ inline size_t owner_plane_bytes(const mi355nufft_plan* p) {
 inline bool use_owner(const mi355nufft_plan* p, int32_t nreps) {
     if (p->ndim != 2 || !use_tiled(p) || !use_fxp(p) || (p->method != 0 && p->method != 2)) return false;
     const int64_t cells = p->nframes * p->nk;
-    if (nreps < kOwnerMinReps || 2 * p->M > cells || (size_t)cells * nreps * p->cx_size() < kOwnerMinBytes)
+    const size_t least = p->bg.B[0] * p->bg.B[1] > 256 ? kOwnerMinBytesLarge : kOwnerMinBytes;
+    if (nreps < kOwnerMinReps || 2 * p->M > cells || (size_t)cells * nreps * p->cx_size() < least)
         return false;
     int segs = 1;
     for (int d = 0; d < 2; ++d) {

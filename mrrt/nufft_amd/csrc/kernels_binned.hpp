@@ -809,6 +809,17 @@ __device__ __forceinline__ cx<T> sample_times_conj_phase(const InterpArgs<T, CK>
 // so only the final sums must fit).  Each tap is rounded to a step of at most
 // 2^-30 1.001 A cmax.  The scale is a power of two, so scaling and unscaling
 // are exact, and the integer sums do not depend on the order of the atomics.
+// WIN (2-D, no coefficient cache, bins of more than 256 cells): A is the largest sum over 2 x 2 blocks of
+// at least J - 1 cells per axis, which hold the first taps of every sample
+// that reaches a cell, instead of the sum over the subproblem; the block sums
+// are integers in units of 2^-20 of the power of two above the largest
+// sample, each sample rounded up.  It keeps the steps of large bins (32 x 32
+// cells: up to ten times the cells of a window) no coarser than those of
+// 16 x 16 bins, whose sum covers 256 cells (adjoint of 200,000 random points
+// on Kd 1024^2 against the float64 tile 1.5e-7, with the sum 2.4e-7, 16 x 16
+// bins 1.5e-7; scatter 22.8 -> 26.0 us).  With 16 x 16 bins the window's
+// second look at the points costs more than its precision is worth (Kd 512^2
+// 16.7 -> 24.5 us, 2.6e-7 -> 2.4e-7).
 // Non-finite samples make the whole tile NaN.  Without FXP (and for
 // complex128) the tile accumulates in float64.
 //
@@ -819,12 +830,15 @@ __device__ __forceinline__ cx<T> sample_times_conj_phase(const InterpArgs<T, CK>
 // coefficient loads run beside the sample reads and no load follows the
 // sum's barriers.  Taken for several repetitions, and for one with the
 // fixed-point tile.
-template <typename T, int NDIM, bool CK, int JMAX, bool FIXED, bool FXP, bool REPS = false, int RC = 1>
+template <typename T, int NDIM, bool CK, int JMAX, bool FIXED, bool FXP, bool REPS = false, int RC = 1,
+          bool WIN = false>
 __global__ __launch_bounds__(256) void spread_tiled_kernel(TiledArgs<T, CK> a) {
     static_assert(!FXP || sizeof(T) == 4, "fixed-point accumulation is for complex64");
+    static_assert(!WIN || (FXP && NDIM == 2 && !REPS), "windowed scale: 2-D fixed point without the cache");
     static_assert(RC == 1 || !REPS, "the coefficient cache is for one repetition per pass");
     extern __shared__ __align__(16) unsigned char smem[];
-    __shared__ float red[4];  // block_sum, at most 256 threads
+    __shared__ float red[4 * RC];  // block_sum and the largest samples, at most 256 threads
+    __shared__ unsigned blk[WIN ? 64 * RC : 1];  // WIN: sample sums of 8 x 8 blocks
     using Acc = typename std::conditional<FXP, int, double>::type;
     // FXP: packed 64-bit cells in 3-D (C3 scatter 0.424 -> 0.411 ms at 2,560
     // points per subproblem, 0.442 -> 0.403 ms at 3,072); two int32 planes in
@@ -872,36 +886,98 @@ __global__ __launch_bounds__(256) void spread_tiled_kernel(TiledArgs<T, CK> a) {
             int km0 = 0, km1 = 0;            // KEEP: indices and samples of points ic and i1
             cx<T> ky0 = yc, ky1 = yc;
             if constexpr (FXP) {
-                float part[RC];
+                float part[RC];  // sum (WIN: largest) of |Re y| + |Im y|
 #pragma unroll
                 for (int k = 0; k < RC; ++k) part[k] = 0.f;
+                auto take = [&](float& acc, cx<T> y) {
+                    const float v = fabsf(y.x) + fabsf(y.y);  // |f| = |y| per component bound (|phase| = 1)
+                    if constexpr (WIN) acc = v > acc || !(v == v) ? v : acc;  // NaN stays
+                    else acc += v;
+                };
                 if (cached) {
                     if (ic < s.end) {
                         yc = ia.in[(int64_t)r0 * ia.M + pc.m];
-                        part[0] = fabsf(yc.x) + fabsf(yc.y);
+                        take(part[0], yc);
                     }
                 } else if (kept) {
                     if (ic < s.end) {
                         km0 = a.bs.perm[ic];
                         ky0 = ia.in[(int64_t)r0 * ia.M + km0];
-                        part[0] = fabsf(ky0.x) + fabsf(ky0.y);
+                        take(part[0], ky0);
                     }
                     if (i1 < s.end) {
                         km1 = a.bs.perm[i1];
                         ky1 = ia.in[(int64_t)r0 * ia.M + km1];
-                        part[0] += fabsf(ky1.x) + fabsf(ky1.y);
+                        take(part[0], ky1);
                     }
                 } else {
                     for (int i = s.start + tid; i < s.end; i += blockDim.x) {
                         const int64_t m = a.bs.perm[i];
 #pragma unroll
                         for (int k = 0; k < RC; ++k)
-                            if (k < rc) {
-                                const cx<T> y = ia.in[(int64_t)(r0 + k) * ia.M + m];
-                                part[k] += fabsf(y.x) + fabsf(y.y);  // |f| = |y| per component bound (|phase| = 1)
-                            }
+                            if (k < rc) take(part[k], ia.in[(int64_t)(r0 + k) * ia.M + m]);
                     }
                 }
+                if constexpr (WIN) {
+                    const int lane = tid & 63, nw = blockDim.x >> 6;
+                    const int b0 = max(ax[0].J - 1, (bg.B[0] + 7) / 8), b1 = max(ax[1].J - 1, (bg.B[1] + 7) / 8);
+                    const float inv0 = 1.0f / (float)b0, inv1 = 1.0f / (float)b1;
+                    int ev[RC];  // the largest sample is below 2^ev
+                    for (int e = tid; e < 64 * RC; e += blockDim.x) blk[e] = 0;
+#pragma unroll
+                    for (int k = 0; k < RC; ++k) {
+#pragma unroll
+                        for (int o = 32; o > 0; o >>= 1) {
+                            const float u = __shfl_xor(part[k], o);
+                            part[k] = u > part[k] || !(u == u) ? u : part[k];
+                        }
+                        if (lane == 0) red[(tid >> 6) * RC + k] = part[k];
+                    }
+                    __syncthreads();
+#pragma unroll
+                    for (int k = 0; k < RC; ++k) {
+                        float v = red[k];
+                        for (int w = 1; w < nw; ++w) {
+                            const float u = red[w * RC + k];
+                            v = u > v || !(u == u) ? u : v;
+                        }
+                        bad[k] = !(v <= 3.4e38f);
+                        ev[k] = 0;
+                        (void)frexpf(bad[k] ? 0.f : v, &ev[k]);
+                    }
+                    auto count = [&](int i, int k, cx<T> y) {
+                        const int l0 = first_tap_mod(a.tms[i], ax[0].J, ax[0].K) - s.o[0];
+                        const int l1 = first_tap_mod(a.tms[ia.M + i], ax[1].J, ax[1].K) - s.o[1];
+                        if (!bad[k])
+                            atomicAdd(&blk[64 * k + 8 * div_small(l1, inv1) + div_small(l0, inv0)],
+                                      (unsigned)ceilf(ldexpf(fabsf(y.x) + fabsf(y.y), 20 - ev[k])) + 1u);
+                    };
+                    if (kept) {
+                        if (ic < s.end) count(ic, 0, ky0);
+                        if (i1 < s.end) count(i1, 0, ky1);
+                    } else {
+                        for (int i = s.start + tid; i < s.end; i += blockDim.x) {
+                            const int64_t m = a.bs.perm[i];
+#pragma unroll
+                            for (int k = 0; k < RC; ++k)
+                                if (k < rc) count(i, k, ia.in[(int64_t)(r0 + k) * ia.M + m]);
+                        }
+                    }
+                    __syncthreads();
+#pragma unroll
+                    for (int k = 0; k < RC; ++k) {
+                        unsigned win = 0;
+                        if (lane < 49) {
+                            const unsigned* q = blk + 64 * k + 8 * (lane / 7) + lane % 7;
+                            win = q[0] + q[1] + q[8] + q[9];
+                        }
+#pragma unroll
+                        for (int o = 32; o > 0; o >>= 1) win = max(win, (unsigned)__shfl_xor((int)win, o));
+                        int e = 0;
+                        (void)frexpf((float)win * a.cmax * 1.001f, &e);  // A = that times 2^(ev - 20)
+                        sh[k] = 51 - ev[k] - e;
+                    }
+                } else {
 #pragma unroll
                 for (int k = 0; k < RC; ++k)
                     if (k < rc) {
@@ -911,8 +987,9 @@ __global__ __launch_bounds__(256) void spread_tiled_kernel(TiledArgs<T, CK> a) {
                         (void)frexpf(A, &e);
                         sh[k] = 31 - e;
                     }
+                }
             }
-            __syncthreads();
+            if constexpr (!WIN) __syncthreads();
             // sample f (times conj(phase)) of repetition r0 + k at point pt
             auto add_sample = [&](int k, const PointTaps<T, CK, JMAX>& pt, cx<T> f) {
                 Acc* tre = tiles + 2 * k * bg.tile;

@@ -727,7 +727,8 @@ int fft_impl(mi355nufft_plan* p, void* grid, int32_t nreps, int direction) {
 namespace mi355host {
 
 // Default bin geometry (autotuned on golden-angle radial and kooshball
-// trajectories): 2-D 16x16 with P = 384 points per subproblem; 3-D 16^3
+// trajectories): 2-D 16x16 with P = 384 points per subproblem, larger on large
+// sparse grids; 3-D 16^3
 // with P = 3072 when the scatter tile is fixed point and no sparse matrix is
 // set, else 16x8x8 with P = 1024; 1-D 512 with P = 512.  Requested sizes
 // override.
@@ -745,6 +746,18 @@ void default_bins(const mi355nufft_plan* p, int B[3], int& P) {
         B[0] = 16;
         B[1] = 16;
         P = 384;
+        // More bins than the 1,024 workgroups and sparse points: bigger bins
+        // leave fewer halos to stage and flush.  Forward and adjoint with
+        // 16x16 / 32x16 / 32x32 bins: Kd 1024^2 and 0.2 points per cell
+        // (radial) 101 / 94 / 88 us, 0.5: 109 / 107 / 121, 0.8: 120 / 132 /
+        // 158; Kd 576^2, 0.2: 63 / 58 / 59; 8 frames x 4 coils of Kd 512^2
+        // 286 / 247 / 219; with 9,953 points on Kd 576^2 50 / 52 / 53; Kd
+        // 512^2 (1,024 bins of 16x16) and 0.79 points per cell 50 / 52 / 60.
+        const int64_t cells = p->nframes * p->nk, bins = cells / 256;
+        if (bins > 1024 && p->M > 16384 && 20 * p->M <= 7 * cells) {
+            B[0] = 32;
+            if (bins >= 2048) B[1] = 32;
+        }
     } else if (fxp_eligible(p) && !p->sparse_bins) {
         // the fixed-point scatter tile of 21^3 cells takes 74 KB of LDS:
         // bigger bins cut the halo and the flush (measured at Kd 256^3:

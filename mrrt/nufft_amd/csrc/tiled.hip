@@ -28,6 +28,10 @@ void launch_tiled(bool adjoint, const TiledArgs<T, CK>& a, unsigned nsub, unsign
             spread = pair ? spread_tiled_kernel<T, NDIM, CK, JMAX, FIXED, true, false, 2>
                           : reps ? spread_tiled_kernel<T, NDIM, CK, JMAX, FIXED, true, true>
                                  : spread_tiled_kernel<T, NDIM, CK, JMAX, FIXED, true, false>;
+    if constexpr (sizeof(T) == 4 && NDIM == 2)  // finer steps in large bins
+        if (a.cmax > 0.f && (pair || !reps) && a.bg.B[0] * a.bg.B[1] > 256)
+            spread = pair ? spread_tiled_kernel<T, NDIM, CK, JMAX, FIXED, true, false, 2, true>
+                          : spread_tiled_kernel<T, NDIM, CK, JMAX, FIXED, true, false, 1, true>;
     auto interp = a.rc > 1 ? interp_tiled_kernel<T, NDIM, CK, JMAX, FIXED, true>
                            : interp_tiled_kernel<T, NDIM, CK, JMAX, FIXED, false>;
     if constexpr (FIXED)  // fused tap sums unless the reference's roundings are asked for
@@ -55,12 +59,13 @@ void launch_tiled(bool adjoint, const TiledArgs<T, CK>& a, unsigned nsub, unsign
         hipLaunchKernelGGL(interp, grid, dim3(threads), lds, s, a);
 }
 
-// Bins of more than one point per cell (and more than one batch) are left to
-// the atomic kernel.  24 frames x 32 coils at 16 x 16 bins: 1334 us with 256,
-// 1376 with 512, 1685 with 1024 and more; 48 frames x 4 coils 533 / 604 / 762.
+// Denser bins are left to the atomic kernel: one batch of points, or half a
+// point per cell of larger bins.  Adjoint of 24 frames x 32 coils: 16x16 bins
+// 2.06 ms with 256, 2.10 with 512, 2.45 with 1024; 32x32 bins 2.35 / 2.20 /
+// 2.30; 4 frames x 32 coils 505 / 511 / 635 us, 511 / 488 / 525.
 inline int owner_heavy(const mi355nufft_plan* p) {
-    const int cells = p->bg.B[0] * p->bg.B[1];
-    return cells > kOwnerBatch ? cells : kOwnerBatch;
+    const int half = p->bg.B[0] * p->bg.B[1] / 2;
+    return half > kOwnerBatch ? half : kOwnerBatch;
 }
 
 template <bool CK, int JMAX, bool FIXED>

@@ -39,7 +39,7 @@ def _points(kind, m, rng):
 def _reps(Kd):
     """The smallest odd count whose grids together pass the size from which
     the path is taken."""
-    return (128 << 20) // (8 * int(np.prod(Kd))) + 1 | 1
+    return (320 << 20) // (8 * int(np.prod(Kd))) + 1 | 1
 
 
 def _samples(reps, m, seed):
@@ -69,9 +69,9 @@ def test_owner_vs_float64_and_oracle(phasing, kind, m, Nd, Kd, Jd, bins):
     got = A.adj(y)
     A.set_kernel_timing(True, count_atomics=True)
     again = A.adj(y)
-    # no atomics on the grid but those of dense bins (more points than cells and than one batch)
+    # no atomics on the grid but those of dense bins (more points than half their cells and than one batch)
     if kind != "edge":
-        dense = kind == "dense" and m // 2 > max(256, int(np.prod(A.plan_info()["bin_size"])))
+        dense = kind == "dense" and m // 2 > max(256, int(np.prod(A.plan_info()["bin_size"])) // 2)
         assert (A.read_flush_atomics() > 0) == dense
     A.set_scatter("float64")
     ref = A.adj(y)
