@@ -347,38 +347,56 @@ inline bool use_owner(const mi355nufft_plan* p, int32_t nreps) {
 }
 
 // The bin sort of the plan's points (p->d_tm, p->M, p->bg) into its binning
-// storage, in six launches: clear the (bin, bank key) counters, count, sum
-// per bin, scan (subproblem table), scatter (perm), and copy tm and the
-// per-sample phase into sorted order.  With gate.p set every launch does
+// storage, in five launches: clear the (bin, bank key) counters, count, sum
+// per bin, scan (subproblem table), and scatter (perm, with tm and the
+// per-sample phase in sorted order).  With gate.p set every launch does
 // nothing unless the check kernel stamped gate.gen (cached sort).
+// The launches in two parts: clear and count (set_points_kernel counts new
+// points itself), and the rest.
+inline int launch_bin_clear(const mi355nufft_plan* p, SortGate gate) {
+    hipLaunchKernelGGL(fill_int_kernel, dim3(nblocks((int64_t)p->bg.nbins * kBanks)), dim3(kBlock), 0, p->stream,
+                       bin_state(p).bkt, (int64_t)p->bg.nbins * kBanks, 0, gate);
+    LAUNCH_CHECK();
+    return MI355NUFFT_OK;
+}
+
+// axis geometry of the plan's taps (no tables)
 template <typename T>
-int launch_bin_sort(const mi355nufft_plan* p, SortGate gate) {
-    const int64_t M = p->M;
-    const int64_t max_sub = max_subproblems(p);
-    const BinState bs = bin_state(p);
+void bin_axes(const mi355nufft_plan* p, AxisGeom (&ax)[3]) {
     InterpArgs<T, false> ia;
     int32_t J[3] = {p->J[0], p->J[1], p->J[2]};
     const void* dummy[3] = {p->d_tab[0], p->d_tab[0], p->d_tab[0]};
-    fill_interp_args<T, false>(ia, p->ndim, p->K, J, p->L, dummy, p->d_tm, M, 1);
-    hipLaunchKernelGGL(fill_int_kernel, dim3(nblocks((int64_t)p->bg.nbins * kBanks)), dim3(kBlock), 0, p->stream,
-                       bs.bkt, (int64_t)p->bg.nbins * kBanks, 0, gate);
-    LAUNCH_CHECK();
-    hipLaunchKernelGGL((bin_count_kernel<T>), dim3(nblocks(M)), dim3(kBlock), 0, p->stream, (const T*)p->d_tm, M,
-                       p->ndim, ia.ax[0], ia.ax[1], ia.ax[2], p->bg, bs, gate);
-    LAUNCH_CHECK();
-    hipLaunchKernelGGL(bin_sum_kernel, dim3(nblocks(p->bg.nbins)), dim3(kBlock), 0, p->stream, bs, p->bg.nbins,
+    fill_interp_args<T, false>(ia, p->ndim, p->K, J, p->L, dummy, p->d_tm, p->M, 1);
+    for (int d = 0; d < 3; ++d) ax[d] = ia.ax[d];
+}
+
+template <typename T>
+int launch_bin_rest(const mi355nufft_plan* p, SortGate gate) {
+    const int64_t M = p->M;
+    const int64_t max_sub = max_subproblems(p);
+    const BinState bs = bin_state(p);
+    hipLaunchKernelGGL(bin_sum_kernel, dim3((unsigned)((p->bg.nbins + kBanks - 1) / kBanks)), dim3(kBlock), 0, p->stream, bs, p->bg.nbins,
                        gate);
     LAUNCH_CHECK();
     hipLaunchKernelGGL(bin_scan_kernel, dim3(1), dim3(1024), 0, p->stream, bs, p->bg.nbins, p->bg.P, (int)max_sub,
                        gate);
     LAUNCH_CHECK();
-    hipLaunchKernelGGL(bin_scatter_kernel, dim3(nblocks(M)), dim3(kBlock), 0, p->stream, M, bs, p->bg.P, gate);
-    LAUNCH_CHECK();
-    hipLaunchKernelGGL((sort_points_kernel<T>), dim3(nblocks(M)), dim3(kBlock), 0, p->stream, (const T*)p->d_tm,
-                       p->has_phase ? (const cx<T>*)p->d_phase : nullptr, M, p->ndim, (const int*)bs.perm,
-                       (T*)p->d_tms, (cx<T>*)p->d_phs, gate);
+    hipLaunchKernelGGL((bin_scatter_kernel<T>), dim3(nblocks(M)), dim3(kBlock), 0, p->stream, (const T*)p->d_tm,
+                       p->has_phase ? (const cx<T>*)p->d_phase : nullptr, M, p->ndim, bs, p->bg.P, (T*)p->d_tms,
+                       (cx<T>*)p->d_phs, gate);
     LAUNCH_CHECK();
     return MI355NUFFT_OK;
+}
+
+template <typename T>
+int launch_bin_sort(const mi355nufft_plan* p, SortGate gate) {
+    RET_IF(launch_bin_clear(p, gate));
+    AxisGeom ax[3];
+    bin_axes<T>(p, ax);
+    hipLaunchKernelGGL((bin_count_kernel<T>), dim3(nblocks(p->M)), dim3(kBlock), 0, p->stream, (const T*)p->d_tm, p->M,
+                       p->ndim, ax[0], ax[1], ax[2], p->bg, bin_state(p), gate);
+    LAUNCH_CHECK();
+    return launch_bin_rest<T>(p, gate);
 }
 
 // bin geometry of the plan's binning request (defaults per ndim; main TU)

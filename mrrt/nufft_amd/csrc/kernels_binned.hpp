@@ -47,7 +47,7 @@ struct BinState {
     int* n_sub;      // (1) number of subproblems
     int* max_count;  // (1) points of the fullest bin
     int* bin_sub;    // (nbins) first subproblem of each bin
-    int* bkt;        // (nbins * kBanks) points per (bin, bank key)
+    int* bkt;        // (nbins * kBanks) points per (bin, bank key), see bkt_slot
     const int64_t* frame_off;  // (nframes + 1) first point of each frame, or null
     int nframes;
 };
@@ -61,6 +61,17 @@ struct BinState {
 // apart.  The same order serves the gather (tile reads) and
 // the scatter (tile atomics).
 constexpr int kBanks = 32;
+
+// Counter of (bin, key) while the points are counted.  The keys of one bin lie
+// in different cache lines (32 bins to a block, key-major), because atomics
+// on one line queue: with a bin's 32 counters in one line, a golden-angle
+// trajectory's centre bins took most of the count's time (205,824 points on
+// Kd 512^2: 22.3 -> 19.5 us).  bin_sum_kernel turns each block to bin-major
+// in place; the bins after the last full block are bin-major from the start.
+__device__ __forceinline__ int bkt_slot(int bin, int key, int nbins) {
+    const int first = bin & ~(kBanks - 1);
+    return first + kBanks <= nbins ? first * kBanks + key * kBanks + (bin - first) : bin * kBanks + key;
+}
 
 // Optional gate of the sort kernels: with p set, a kernel does nothing unless
 // *p == gen.  A check kernel earlier in the stream stamps gen when the points
@@ -80,16 +91,13 @@ __device__ __forceinline__ int first_tap_mod(T t, int J, int K) {
     return pos_mod(first_tap(t, J), K);
 }
 
+// Bin and bank key of point m at t, and its rank among the points of both.
 template <typename T>
-__global__ __launch_bounds__(256) void bin_count_kernel(const T* __restrict__ tm, int64_t M, int ndim,
-                                                        AxisGeom a0, AxisGeom a1, AxisGeom a2, BinGeom bg,
-                                                        BinState bs, SortGate gate) {
-    const int64_t m = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (m >= M || gate_closed(gate)) return;
-    const AxisGeom ax[3] = {a0, a1, a2};
+__device__ __forceinline__ void bin_point(int64_t m, const T (&t)[3], int ndim, const AxisGeom* ax, const BinGeom& bg,
+                                          const BinState& bs) {
     int bin = 0, mul = 1, base = 0, tmul = 1;
     for (int d = 0; d < ndim; ++d) {
-        const int k0 = first_tap_mod(tm[(int64_t)d * M + m], ax[d].J, ax[d].K);
+        const int k0 = first_tap_mod(t[d], ax[d].J, ax[d].K);
         const int b = k0 / bg.B[d];
         bin += b * mul;
         mul *= bg.nb[d];
@@ -105,23 +113,97 @@ __global__ __launch_bounds__(256) void bin_count_kernel(const T* __restrict__ tm
         }
         bin += lo * bg.nbins_frame;
     }
-    const int slot = bin * kBanks + (base & (kBanks - 1));
-    bs.bin_of[m] = slot;
-    bs.rank[m] = atomicAdd(&bs.bkt[slot], 1);
+    const int key = base & (kBanks - 1);
+    bs.bin_of[m] = bin * kBanks + key;
+    bs.rank[m] = atomicAdd(&bs.bkt[bkt_slot(bin, key, bg.nbins)], 1);
 }
 
-// counts[b] = points of bin b (sum over its bank keys)
-static __global__ __launch_bounds__(256) void bin_sum_kernel(BinState bs, int nbins, SortGate gate) {
-    const int b = blockIdx.x * blockDim.x + threadIdx.x;
-    if (b >= nbins || gate_closed(gate)) return;
-    const int4* q = reinterpret_cast<const int4*>(bs.bkt + (int64_t)b * kBanks);
-    int c = 0;
-#pragma unroll
-    for (int k = 0; k < kBanks / 4; ++k) {
-        const int4 v = q[k];
-        c += v.x + v.y + v.z + v.w;
+template <typename T>
+__global__ __launch_bounds__(256) void bin_count_kernel(const T* __restrict__ tm, int64_t M, int ndim,
+                                                        AxisGeom a0, AxisGeom a1, AxisGeom a2, BinGeom bg,
+                                                        BinState bs, SortGate gate) {
+    const int64_t m = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (m >= M || gate_closed(gate)) return;
+    const AxisGeom ax[3] = {a0, a1, a2};
+    T t[3] = {0, 0, 0};
+    for (int d = 0; d < ndim; ++d) t[d] = tm[(int64_t)d * M + m];
+    bin_point<T>(m, t, ndim, ax, bg, bs);
+}
+
+// Per-sample set-up of new points and, with count set, their bin count.
+//   tm[d*M + m] = (T)omega / (T)(2 pi / K_d)  in T (_nufft.py:338-342 after
+//   the cast of omega at :315).  For float the quotient is formed in double
+//   and rounded once, which equals the correctly rounded float quotient.
+//   phase_mode 1: phase_after = exp(i omega . shift) (_nufft.py:717-724) from
+//   the uncast omega, dot in float32 (dot_single) or float64;
+//   phase_mode 2: phase_shift = exp(i omega_T . n_shift) in float64
+//   (_nufft.py:898-901).
+template <typename T, typename W>
+__global__ __launch_bounds__(256) void set_points_kernel(const W* __restrict__ omega, int64_t M, int64_t sm,
+                                                         int64_t sd, int ndim, double g0, double g1, double g2,
+                                                         T* __restrict__ tm, cx<T>* __restrict__ phase,
+                                                         int phase_mode, double s0, double s1, double s2,
+                                                         int dot_single, int count, AxisGeom a0, AxisGeom a1,
+                                                         AxisGeom a2, BinGeom bg, BinState bs) {
+    const int64_t m = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (m >= M) return;
+    const double gam[3] = {g0, g1, g2};
+    const double sh[3] = {s0, s1, s2};
+    W w[3] = {0, 0, 0};
+    T wr[3] = {0, 0, 0}, t[3] = {0, 0, 0};
+    for (int d = 0; d < ndim; ++d) {
+        w[d] = omega[m * sm + (int64_t)d * sd];
+        wr[d] = (T)w[d];
+        const T gt = (T)gam[d];
+        t[d] = (T)((double)wr[d] / (double)gt);
+        tm[(int64_t)d * M + m] = t[d];
     }
-    bs.counts[b] = c;
+    if (count) {
+        const AxisGeom ax[3] = {a0, a1, a2};
+        bin_point<T>(m, t, ndim, ax, bg, bs);
+    }
+    if (phase_mode == 1 && dot_single) {
+        float a = (float)w[0] * (float)sh[0];
+        for (int d = 1; d < ndim; ++d) a = a + (float)w[d] * (float)sh[d];
+        double sd_, cd_;
+        sincos((double)a, &sd_, &cd_);
+        phase[m] = mkcx<T>((T)(float)cd_, (T)(float)sd_);
+    } else if (phase_mode) {
+        double acc = phase_mode == 1 ? (double)w[0] * sh[0] : (double)wr[0] * sh[0];
+        for (int d = 1; d < ndim; ++d) acc = acc + (phase_mode == 1 ? (double)w[d] : (double)wr[d]) * sh[d];
+        double s, c;
+        sincos(acc, &s, &c);
+        phase[m] = mkcx<T>((T)c, (T)s);
+    }
+}
+
+// counts[b] = points of bin b (sum over its bank keys), and the counters of
+// each full block of 32 bins from key-major to bin-major.  One workgroup of 256
+// threads per 32 bins, four counters per thread.
+static __global__ __launch_bounds__(256) void bin_sum_kernel(BinState bs, int nbins, SortGate gate) {
+    __shared__ int t[kBanks][kBanks + 1];
+    if (gate_closed(gate)) return;  // uniform over the workgroup, before the barrier
+    const int b0 = blockIdx.x * kBanks, tid = threadIdx.x;
+    const bool full = b0 + kBanks <= nbins;
+    const int row = tid / 8, col = 4 * (tid % 8);  // of the block as it lies in memory
+    int4* q = reinterpret_cast<int4*>(bs.bkt + (int64_t)b0 * kBanks) + tid;
+    if (full || b0 + row < nbins) {
+        const int4 v = *q;
+        const int c[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            if (full) t[col + u][row] = c[u];  // row: key, col: bin
+            else t[row][col + u] = c[u];
+        }
+    }
+    __syncthreads();
+    if (full) *q = make_int4(t[row][col], t[row][col + 1], t[row][col + 2], t[row][col + 3]);
+    if (tid < kBanks && b0 + tid < nbins) {
+        int c = 0;
+#pragma unroll
+        for (int k = 0; k < kBanks; ++k) c += t[tid][k];
+        bs.counts[b0 + tid] = c;
+    }
 }
 
 // One workgroup of 1024 threads: exclusive scans of the bin counts and of the
@@ -192,7 +274,13 @@ static __global__ __launch_bounds__(1024) void bin_scan_kernel(BinState bs, int 
 // levels a stride of ns would otherwise meet only 32 / gcd(ns, 32) keys
 // (a subproblem of a bin with ns = 16 sees two, and its lanes queue on two
 // LDS banks); rotated, consecutive levels supply the other residues.
-static __global__ __launch_bounds__(256) void bin_scatter_kernel(int64_t M, BinState bs, int P, SortGate gate) {
+// tm and the per-sample phase are copied into that order beside it, so the
+// tiled kernels read them coalesced instead of through perm.
+template <typename T>
+__global__ __launch_bounds__(256) void bin_scatter_kernel(const T* __restrict__ tm, const cx<T>* __restrict__ phase,
+                                                          int64_t M, int ndim, BinState bs, int P,
+                                                          T* __restrict__ tms, cx<T>* __restrict__ phs,
+                                                          SortGate gate) {
     const int64_t m = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (m >= M || gate_closed(gate)) return;
     const int slot = bs.bin_of[m];
@@ -217,7 +305,10 @@ static __global__ __launch_bounds__(256) void bin_scatter_kernel(int64_t M, BinS
     }
     const int q = c / ns, rem = c - q * ns;
     const int j = pos % ns;
-    bs.perm[bs.bin_start[bin] + j * q + min(j, rem) + pos / ns] = (int)m;
+    const int64_t i = bs.bin_start[bin] + j * q + min(j, rem) + pos / ns;
+    bs.perm[i] = (int)m;
+    for (int d = 0; d < ndim; ++d) tms[(int64_t)d * M + i] = tm[(int64_t)d * M + m];
+    if (phase) phs[i] = phase[m];
 }
 
 static __global__ __launch_bounds__(256) void fill_int_kernel(int* __restrict__ p, int64_t n, int v, SortGate gate) {
@@ -264,20 +355,6 @@ struct TiledArgs {
     unsigned long long* flush_count;  // scatter: non-null adds the flush's global atomic lane operations
     int flush_slots;                  // power of two: workgroup b adds to flush_count[b % flush_slots]
 };
-
-// Copy tm and the per-sample phase into sorted (bin) order, so the tiled
-// kernels read them coalesced instead of through perm.
-template <typename T>
-__global__ __launch_bounds__(256) void sort_points_kernel(const T* __restrict__ tm, const cx<T>* __restrict__ phase,
-                                                          int64_t M, int ndim, const int* __restrict__ perm,
-                                                          T* __restrict__ tms, cx<T>* __restrict__ phs,
-                                                          SortGate gate) {
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= M || gate_closed(gate)) return;
-    const int64_t m = perm[i];
-    for (int d = 0; d < ndim; ++d) tms[(int64_t)d * M + i] = tm[(int64_t)d * M + m];
-    if (phase) phs[i] = phase[m];
-}
 
 struct Sub {
     int start, end;

@@ -1,6 +1,6 @@
 // Elementwise kernels around the FFT: deapodization + zero-pad onto the
 // oversampled grid, the phase_before multiply, crop + scale + deapodization,
-// grid zeroing, and the per-sample set-up (tm and per-sample phase).
+// and grid zeroing.
 #pragma once
 
 #include "device_common.hpp"
@@ -150,59 +150,6 @@ template <typename T>
 __global__ __launch_bounds__(256) void zero_kernel(cx<T>* __restrict__ p, int64_t n) {
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i < n) p[i] = mkcx<T>((T)0, (T)0);
-}
-
-// Per-sample set-up.
-//   tm[d*M + m] = (T)omega / (T)(2 pi / K_d)  in T (_nufft.py:338-342 after
-//   the cast of omega at :315).  For float the quotient is formed in double
-//   and rounded once, which equals the correctly rounded float quotient.
-//   phase_mode 1: phase_after = exp(i omega . shift) (_nufft.py:717-724) from
-//   the uncast omega, dot in float32 (dot_single) or float64;
-//   phase_mode 2: phase_shift = exp(i omega_T . n_shift) in float64
-//   (_nufft.py:898-901).
-template <typename T, typename W>
-__global__ __launch_bounds__(256) void set_points_kernel(const W* __restrict__ omega, int64_t M, int64_t sm,
-                                                         int64_t sd, int ndim, double g0, double g1, double g2,
-                                                         T* __restrict__ tm, cx<T>* __restrict__ phase,
-                                                         int phase_mode, double s0, double s1, double s2,
-                                                         int dot_single) {
-    const int64_t m = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (m >= M) return;
-    const double gam[3] = {g0, g1, g2};
-    const double sh[3] = {s0, s1, s2};
-    W w[3] = {0, 0, 0};
-    T wr[3] = {0, 0, 0};
-    for (int d = 0; d < ndim; ++d) {
-        w[d] = omega[m * sm + (int64_t)d * sd];
-        wr[d] = (T)w[d];
-        const T gt = (T)gam[d];
-        tm[(int64_t)d * M + m] = (T)((double)wr[d] / (double)gt);
-    }
-    if (phase_mode == 1) {
-        double acc;
-        if (dot_single) {
-            float a = (float)w[0] * (float)sh[0];
-            for (int d = 1; d < ndim; ++d) a = a + (float)w[d] * (float)sh[d];
-            float sf, cf;
-            double sd_, cd_;
-            sincos((double)a, &sd_, &cd_);
-            sf = (float)sd_;
-            cf = (float)cd_;
-            phase[m] = mkcx<T>((T)cf, (T)sf);
-            return;
-        }
-        acc = (double)w[0] * sh[0];
-        for (int d = 1; d < ndim; ++d) acc = acc + (double)w[d] * sh[d];
-        double s, c;
-        sincos(acc, &s, &c);
-        phase[m] = mkcx<T>((T)c, (T)s);
-    } else if (phase_mode == 2) {
-        double acc = (double)wr[0] * sh[0];
-        for (int d = 1; d < ndim; ++d) acc = acc + (double)wr[d] * sh[d];
-        double s, c;
-        sincos(acc, &s, &c);
-        phase[m] = mkcx<T>((T)c, (T)s);
-    }
 }
 
 }  // namespace mi355

@@ -841,9 +841,10 @@ int grow(mi355nufft_plan* p, Tp** buf, int64_t& cap, int64_t need, int64_t per) 
     return MI355NUFFT_OK;
 }
 
-template <typename T>
-int bin_points_impl(mi355nufft_plan* p) {
+// Bin geometry and storage of the plan's points; *use: the points get sorted.
+int prepare_bins(mi355nufft_plan* p, bool* use) {
     p->binned = 0;
+    *use = false;
     if (p->method == 1 || p->M == 0) return MI355NUFFT_OK;
     setup_bin_geom(p);
     if (p->method == 4 && !p->reduce_ok)
@@ -875,6 +876,15 @@ int bin_points_impl(mi355nufft_plan* p) {
             return fail(MI355NUFFT_ENOMEM, "sorted points storage for M=%lld", (long long)M);
         p->sorted_cap = M;
     }
+    *use = true;
+    return MI355NUFFT_OK;
+}
+
+template <typename T>
+int bin_points_impl(mi355nufft_plan* p) {
+    bool use = false;
+    RET_IF(prepare_bins(p, &use));
+    if (!use) return MI355NUFFT_OK;
     RET_IF(launch_bin_sort<T>(p, SortGate{nullptr, 0}));
     p->binned = 1;
     return MI355NUFFT_OK;
@@ -1056,9 +1066,9 @@ int need_points(const mi355nufft_plan* p) {
 // (tm, table pointers, grid) on every call, like the C kernels they replace.
 // They run the tiled kernels on a bin sort of tm that is cached: a check
 // kernel compares tm with the copy the cached sort was made from and stamps
-// a per-call generation number when anything differs; the six sort launches
+// a per-call generation number when anything differs; the five sort launches
 // are gated on that stamp, so an unchanged tm costs one compare pass and
-// six empty launches, and a changed one (even in place, at the same address)
+// five empty launches, and a changed one (even in place, at the same address)
 // is re-sorted within the same call.  The host never reads anything back.
 // Geometries whose scatter tile does not fit the LDS budget run the
 // global-memory kernels, which need no workspace.
@@ -1530,10 +1540,22 @@ int mi355nufft_set_points_frames(mi355nufft_plan* p, const void* omega, int omeg
     double sh[3] = {0, 0, 0};
     if (shift)
         for (int d = 0; d < p->ndim; ++d) sh[d] = shift[d];
+    // a refused binning still leaves the points set, as without it
+    bool sort = false;
+    const int rc = prepare_bins(p, &sort);
+    if (sort) RET_IF(launch_bin_clear(p, SortGate{nullptr, 0}));
+    AxisGeom ax[3] = {};
+    BinState bs = {};
+    if (sort) {
+        if (p->precision) bin_axes<double>(p, ax);
+        else bin_axes<float>(p, ax);
+        bs = bin_state(p);
+    }
 #define SP_LAUNCH(T, W)                                                                                     \
     hipLaunchKernelGGL((set_points_kernel<T, W>), dim3(nblocks(M)), dim3(kBlock), 0, p->stream,             \
                        (const W*)omega, M, stride_m, stride_d, p->ndim, gam[0], gam[1], gam[2], (T*)p->d_tm, \
-                       (cx<T>*)p->d_phase, phase_mode, sh[0], sh[1], sh[2], dot_single)
+                       (cx<T>*)p->d_phase, phase_mode, sh[0], sh[1], sh[2], dot_single, sort ? 1 : 0, ax[0], \
+                       ax[1], ax[2], p->bg, bs)
     if (p->precision == 0) {
         if (omega_double) SP_LAUNCH(float, double);
         else SP_LAUNCH(float, float);
@@ -1543,7 +1565,11 @@ int mi355nufft_set_points_frames(mi355nufft_plan* p, const void* omega, int omeg
     }
 #undef SP_LAUNCH
     LAUNCH_CHECK();
-    return bin_points(p);
+    if (!sort) return rc;
+    RET_IF(p->precision ? launch_bin_rest<double>(p, SortGate{nullptr, 0})
+                        : launch_bin_rest<float>(p, SortGate{nullptr, 0}));
+    p->binned = 1;
+    return MI355NUFFT_OK;
 }
 
 int mi355nufft_set_binning(mi355nufft_plan* p, const int32_t* bin_size, int32_t max_points, int method) {
