@@ -314,7 +314,7 @@ inline int fixed_j(int ndim, const int32_t* Jd) {
 // fixed-point tiles whose geometry it takes (the bins that reach one owned
 // tile fit its list, the periodic range of a tile does not meet itself) with
 // grids that together are too large for the caches and at most one point per
-// two cells; the atomic kernel keeps up longer with bins larger than 16x16.
+// two cells; the atomic kernel keeps up longer with bins of 32x32.
 // Whole adjoints, owner / atomic: 32x32 bins, 24 frames x 32 coils of Kd
 // 512^2 (1.6 GB) 2.31 / 3.12 ms, 12 x 16 (384 MB) 694 / 753 us, 24 x 6 (288
 // MB) 578 / 581, 8 x 16 (256 MB) 531 / 509; 16x16 bins, 128 coils of one
@@ -334,7 +334,7 @@ inline size_t owner_plane_bytes(const mi355nufft_plan* p) {
 inline bool use_owner(const mi355nufft_plan* p, int32_t nreps) {
     if (p->ndim != 2 || !use_tiled(p) || !use_fxp(p) || (p->method != 0 && p->method != 2)) return false;
     const int64_t cells = p->nframes * p->nk;
-    const size_t least = p->bg.B[0] * p->bg.B[1] > 256 ? kOwnerMinBytesLarge : kOwnerMinBytes;
+    const size_t least = p->bg.B[0] * p->bg.B[1] > 512 ? kOwnerMinBytesLarge : kOwnerMinBytes;
     if (nreps < kOwnerMinReps || 2 * p->M > cells || (size_t)cells * nreps * p->cx_size() < least)
         return false;
     int segs = 1;

@@ -746,15 +746,16 @@ void default_bins(const mi355nufft_plan* p, int B[3], int& P) {
         B[0] = 16;
         B[1] = 16;
         P = 384;
-        // More bins than the 1,024 workgroups and sparse points: bigger bins
+        // As many bins as the 1,024 workgroups and sparse points: bigger bins
         // leave fewer halos to stage and flush.  Forward and adjoint with
         // 16x16 / 32x16 / 32x32 bins: Kd 1024^2 and 0.2 points per cell
         // (radial) 101 / 94 / 88 us, 0.5: 109 / 107 / 121, 0.8: 120 / 132 /
         // 158; Kd 576^2, 0.2: 63 / 58 / 59; 8 frames x 4 coils of Kd 512^2
-        // 286 / 247 / 219; with 9,953 points on Kd 576^2 50 / 52 / 53; Kd
-        // 512^2 (1,024 bins of 16x16) and 0.79 points per cell 50 / 52 / 60.
+        // 286 / 247 / 219; Kd 512^2 (1,024 bins of 16x16), 0.25 random
+        // points per cell 44 / 42 / 44, 8 coils 132 / 115 / 108, 0.79 points
+        // per cell 50 / 52 / 60; with 9,953 points on Kd 576^2 50 / 52 / 53.
         const int64_t cells = p->nframes * p->nk, bins = cells / 256;
-        if (bins > 1024 && p->M > 16384 && 20 * p->M <= 7 * cells) {
+        if (bins >= 1024 && p->M > 16384 && 20 * p->M <= 7 * cells) {
             B[0] = 32;
             if (bins >= 2048) B[1] = 32;
         }

@@ -211,9 +211,11 @@ int run_grad(mi355nufft_plan* p, const void* grid, const void* w, void* grad, in
         g.shift[d] = (T)p->shift[d];
     }
     const unsigned nsub = tiled_grid(p);
-    {  // repetitions staged per pass, as in the gather
-        const size_t chunk_lds = p->lds_limit < kRepChunkLds ? p->lds_limit : kRepChunkLds;
-        int rc = (int)(chunk_lds / gather_tile_bytes(p));
+    {  // repetitions staged per pass, as in the gather; up to 52 KB (three
+       // workgroups per CU) where that takes all of them at once
+        const size_t chunk = p->lds_limit < kRepChunkLds ? p->lds_limit : kRepChunkLds;
+        const size_t one = gather_tile_bytes(p);
+        int rc = (int)((nreps <= kMaxRepChunk && nreps * one <= (chunk * 13) / 10 ? nreps * one : chunk) / one);
         rc = rc < kMaxRepChunk ? rc : kMaxRepChunk;
         rc = rc < nreps ? rc : nreps;
         a.rc = rc > 1 ? rc : 1;

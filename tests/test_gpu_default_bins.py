@@ -15,9 +15,10 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("Kd,m,bins", [
-    ((512, 512), 20000, (16, 16)),      # 1,024 bins
-    ((528, 512), 16384, (16, 16)),      # few points
-    ((528, 512), 16385, (32, 16)),
+    ((504, 512), 20000, (16, 16)),      # 1,008 bins' worth of cells
+    ((512, 512), 16384, (16, 16)),      # few points
+    ((512, 512), 16385, (32, 16)),
+    ((512, 512), 100000, (16, 16)),     # 0.38 points per cell
     ((736, 720), 40000, (32, 32)),
     ((736, 720), 200000, (16, 16)),     # 0.38 points per cell
 ])
