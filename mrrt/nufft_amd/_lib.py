@@ -124,6 +124,15 @@ def i64arr(vals):
     return (ctypes.c_int64 * len(vals))(*[int(v) for v in vals])
 
 
+_I64 = tuple(ctypes.c_int64 * n for n in range(8))
+
+
+def strides(t):
+    """Element strides of a tensor (at most seven axes) as a C array."""
+    st = t.stride()
+    return _I64[len(st)](*st)
+
+
 def i32arr(vals):
     return (ctypes.c_int32 * len(vals))(*[int(v) for v in vals])
 
