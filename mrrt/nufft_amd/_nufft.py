@@ -474,7 +474,8 @@ class NufftBase(object):
         return self._tm_dev_cache
 
     def _sync_stream(self):
-        # the handle without a Stream object (2.5 us of a 17 us call)
+        # the handle without a Stream object: 0.1 instead of 1.8 us of host time
+        # per call
         index = self.device.index
         s = torch._C._cuda_getCurrentRawStream(torch.cuda.current_device() if index is None else index)
         if s != self._stream:
