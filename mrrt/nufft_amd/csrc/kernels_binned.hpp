@@ -988,11 +988,25 @@ __global__ __launch_bounds__(256) void spread_tiled_kernel(TiledArgs<T, CK> a) {
                         take(part[0], ky1);
                     }
                 } else {
-                    for (int i = s.start + tid; i < s.end; i += blockDim.x) {
-                        const int64_t m = a.bs.perm[i];
+                    // U indices, then U samples in flight per thread: one at
+                    // a time, a 3-D subproblem of 3,072 points waits for two
+                    // dependent loads twelve times (measured with the loop
+                    // below)
+                    constexpr int U = NDIM == 3 && sizeof(T) == 4 ? 6 : 1;
+                    for (int i = s.start + tid; i < s.end; i += U * blockDim.x) {
+                        int m[U];
 #pragma unroll
-                        for (int k = 0; k < RC; ++k)
-                            if (k < rc) take(part[k], ia.in[(int64_t)(r0 + k) * ia.M + m]);
+                        for (int u = 0; u < U; ++u) m[u] = i + u * blockDim.x < s.end ? a.bs.perm[i + u * blockDim.x] : -1;
+#pragma unroll
+                        for (int k = 0; k < RC; ++k) {
+                            if (k >= rc) break;
+                            cx<T> y[U];
+#pragma unroll
+                            for (int u = 0; u < U; ++u)
+                                y[u] = m[u] >= 0 ? ia.in[(int64_t)(r0 + k) * ia.M + m[u]] : mkcx<T>((T)0, (T)0);
+#pragma unroll
+                            for (int u = 0; u < U; ++u) take(part[k], y[u]);
+                        }
                     }
                 }
                 if constexpr (WIN) {
@@ -1105,6 +1119,41 @@ __global__ __launch_bounds__(256) void spread_tiled_kernel(TiledArgs<T, CK> a) {
                         point_taps_pre<T, NDIM, CK, JMAX, FIXED>(a, ax, s, t, u ? km1 : km0, ph, pt);
                         add_sample(0, pt, times_conj_phase<T, CK, JMAX>(u ? ky1 : ky0, pt, a.phs));
                     }
+                }
+            } else if constexpr (NDIM == 3 && RC == 1 && !REPS && sizeof(T) == 4) {
+                // The next point's sample, position and phase and the index
+                // after it load while this one's taps are added: the two
+                // workgroups per CU that fit (a tile of 21^3 cells is 74 KB)
+                // do not cover the two dependent loads.  128^3, 2,097,152 points: 426 -> 410 us;
+                // 500,003 points on 192x180x120: 170 -> 167.  Double, which
+                // gets slower with it, 200 -> 206: not there.
+                int i = s.start + tid;
+                const int step = blockDim.x;
+                const cx<T>* yin = ia.in + (int64_t)r0 * ia.M;
+                T tn[3] = {0, 0, 0};
+                cx<T> pn = mkcx<T>((T)1, (T)0), yn = mkcx<T>((T)0, (T)0);
+                int m1 = 0;  // index of point i + step
+                if (i < s.end) {
+                    yn = yin[a.bs.perm[i]];
+                    if (i + step < s.end) m1 = a.bs.perm[i + step];
+#pragma unroll
+                    for (int d = 0; d < 3; ++d) tn[d] = a.tms[(int64_t)d * ia.M + i];
+                    if (a.phs) pn = a.phs[i];
+                }
+                for (; i < s.end; i += step) {
+                    const T tc[3] = {tn[0], tn[1], tn[2]};
+                    const cx<T> pc3 = pn, y3 = yn;
+                    const int in = i + step;
+                    if (in < s.end) {
+                        yn = yin[m1];
+                        if (in + step < s.end) m1 = a.bs.perm[in + step];
+#pragma unroll
+                        for (int d = 0; d < 3; ++d) tn[d] = a.tms[(int64_t)d * ia.M + in];
+                        if (a.phs) pn = a.phs[in];
+                    }
+                    PointTaps<T, CK, JMAX> pt;
+                    point_taps_pre<T, NDIM, CK, JMAX, FIXED>(a, ax, s, tc, 0, pc3, pt);
+                    add_sample(0, pt, times_conj_phase<T, CK, JMAX>(y3, pt, a.phs));
                 }
             } else {
                 for (int i = s.start + tid; i < s.end; i += blockDim.x) {
