@@ -6,12 +6,16 @@
 //
 // What it replaces: the tile per bin subproblem (spread_tiled_kernel) adds
 // its halo, and cells shared between subproblems, to the grid with one
-// global float atomic per component, which needs a cleared grid.  Where the
-// grids of a call do not fit the last-level cache, every such atomic is a
-// read-modify-write in HBM, and the clear is one more pass over the grid.
+// global float atomic per component, which needs a cleared grid.
 // Here points near a tile's edge are evaluated by up to four workgroups
 // ((32 + 5)^2 / 32^2 = 1.34 evaluations per point at J = 6), and the grid is
-// written in whole lines with no read and no clear.
+// written in whole lines with no clear.  24 frames x 32 coils of Kd 512^2
+// (64x32 bins): 93.7 M -> 22.8 M global atomics per scatter and 1.85 -> 1.63
+// ms.  The bytes do not fall (2.10 -> 2.62 GB by the HBM counters: samples are
+// read again for each tile they reach, and the atomic kernel skips empty
+// cells); what falls is the atomics and, because nothing has to be left zero,
+// the stores of the inverse FFT passes (columns 626 -> 490 us, crop 386 ->
+// 250 us).
 //
 // Points of bins with more than `heavy` points are left to the atomic kernel,
 // launched afterwards on top of what this one stored, so that a dense
