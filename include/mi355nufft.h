@@ -125,7 +125,9 @@ int64_t mi355nufft_num_points(const mi355nufft_plan *plan);
  * Bin geometry and kernel choice for the interpolation stages (no counterpart
  * in the reference, whose kernels run one thread per sample unsorted).
  *   bin_size    ndim bin sizes in grid points (NULL or 0 entries: defaults
- *               2-D 16x16; 3-D 16x16x16 for complex64 with the fixed-point
+ *               2-D 16x16, or 32x16 / 32x32 with more than 16,384 points, at
+ *               most 0.35 per grid point, from 1,024 / 2,048 bins of 16x16 on;
+ *               3-D 16x16x16 for complex64 with the fixed-point
  *               scatter tile and no sparse matrix set, else 16x8x8; 1-D
  *               512; the scatter tile, 8 bytes
  *               per point in fixed point or 16 in float64 (see
@@ -285,8 +287,9 @@ int mi355nufft_crop_deapod(mi355nufft_plan *plan, const void *grid, void *x,
  * Image -> oversampled grid, grid = fftn(x * sn, Kd) for nimg images (x and
  * xs as mi355nufft_forward, nimg = frames * reps): _nufft.py:1326-1331.
  * phase_before (:1371) is not applied here; the gather applies it.  Grids
- * whose every K_d is a power of two in 16..2048 (16..1024 for complex128)
- * run pruned FFT passes that
+ * whose every K_d is a power of two in 16..2048 (16..1024 for complex128), and
+ * 3-D grids and 2-D grids of more than 96^2 points whose K_d have the prime
+ * factors 2, 3, 5 and 7 only, run pruned FFT passes that
  * read only the image (deapodization fused into the first pass); other
  * grids run mi355nufft_deapod_pad + mi355nufft_fft.
  */
@@ -296,7 +299,7 @@ int mi355nufft_forward_grid(mi355nufft_plan *plan, const void *x,
 /*
  * Oversampled grid -> image, x = ifftn(grid)[:Nd] * scale * conj(sn):
  * _nufft.py:1524-1572 (conj(phase_before) of :1519 is applied by the
- * scatter).  The grid is overwritten.  Power-of-two grids as above run
+ * scatter).  The grid is overwritten.  The grids named above run
  * pruned passes that write only the image rows (crop and deapodization
  * fused into the last pass); others mi355nufft_fft + mi355nufft_crop_deapod.
  */

@@ -432,7 +432,9 @@ class NufftBase(object):
     def set_fft(self, method="auto"):
         """FFT of the transforms: "auto" (pruned passes fused with the
         deapodization for power-of-two grids, 16 <= K <= 2048, complex128
-        K <= 1024) or "rocfft"."""
+        K <= 1024, and for 3-D grids and 2-D grids of more than 96^2 points
+        with prime factors 2, 3, 5 and 7 only; rocFFT for others) or
+        "rocfft"."""
         m = {"auto": 0, "rocfft": 1}[method]
         _lib.check(self._lib.mi355nufft_set_fft(self._plan, m))
 

@@ -2,17 +2,19 @@
 
 ``NufftFrames`` holds one plan for F frames, each frame with its own
 sampling points (uneven sample counts M_f) and C coil images.  A transform
-is three launches plus rocFFT for all F*C images at once:
+is a few launches for all F*C images at once:
 
-* deapodization + zero-pad of all F*C images (one kernel),
-* one batched rocFFT of the F*C oversampled grids,
-* one persistent tiled gather (or scatter) over every (frame, subproblem)
-  work item, each coil reusing the per-point coefficients.
+* FFT passes over all F*C images with the deapodization and zero-pad (or the
+  crop) fused in, one per axis (rocFFT where the grid has no fused passes),
+* one tiled gather (or scatter) over every (frame, subproblem) work item,
+  each coil reusing the per-point coefficients; the scatter of grids too large
+  for the caches writes each grid cell from the workgroup that owns it.
 
 ``capture()`` records the forward and adjoint into HIP graphs (torch's
 CUDAGraph API on ROCm) so that a transform is a single graph launch.  Its
-eager warm-up calls leave the plan's adjoint grid all zero, so the captured
-adjoint has no grid-clearing pass; every replay leaves the grid zero again.
+eager warm-up calls leave the plan's adjoint grid all zero (where the scatter
+adds to it), so the captured adjoint has no grid-clearing pass; every replay
+leaves that grid zero again.
 The reference has no batched path: its repetitions are a Python loop of
 one kernel launch per repetition (mrrt/nufft/_nufft.py:1069-1084, :1181-1189).
 """
@@ -104,7 +106,7 @@ class NufftFrames(object):
         s = torch.cuda.Stream(device=self.device)
         s.wait_stream(torch.cuda.current_stream(self.device))
         with torch.cuda.stream(s):
-            for _ in range(2):  # creates the rocFFT plans and work buffers outside capture
+            for _ in range(2):  # creates FFT plans, grids and work buffers outside capture
                 self.forward(x, out=y)
                 self.adjoint(y, out=xa)
         torch.cuda.current_stream(self.device).wait_stream(s)
