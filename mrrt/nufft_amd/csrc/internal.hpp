@@ -287,6 +287,13 @@ inline int jmax_of(int ndim, const int32_t* Jd) {
     return j <= 4 ? 4 : (j <= 8 ? 8 : 16);
 }
 
+// Points per subproblem up to which the windowed fixed-point scale holds: its
+// 32-bit block sums take at most 2^20 + 1 per sample, and 4,095 (2^20 + 1) is
+// the last multiple below 2^32.  Larger subproblems use the sum over all
+// their samples.
+constexpr int kWindowMaxP = 4095;
+static_assert(kWindowMaxP * ((1ull << 20) + 1) < (1ull << 32), "32-bit block sums");
+
 // Repetitions (coils) whose tiles one tiled launch stages together, and the
 // LDS they may take (more per workgroup costs occupancy: at 24 frames x 32
 // coils of 512^2 grids the gather took 1.18 ms with 64 KB, 0.81 ms with

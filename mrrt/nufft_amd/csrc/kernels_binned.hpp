@@ -886,11 +886,13 @@ __device__ __forceinline__ cx<T> sample_times_conj_phase(const InterpArgs<T, CK>
 // so only the final sums must fit).  Each tap is rounded to a step of at most
 // 2^-30 1.001 A cmax.  The scale is a power of two, so scaling and unscaling
 // are exact, and the integer sums do not depend on the order of the atomics.
-// WIN (2-D, no coefficient cache, bins of more than 256 cells): A is the largest sum over 2 x 2 blocks of
+// WIN (2-D, no coefficient cache, bins of more than 256 cells, at most 4,095
+// points per subproblem): A is the largest sum over 2 x 2 blocks of
 // at least J - 1 cells per axis, which hold the first taps of every sample
 // that reaches a cell, instead of the sum over the subproblem; the block sums
-// are integers in units of 2^-20 of the power of two above the largest
-// sample, each sample rounded up.  It keeps the steps of large bins (32 x 32
+// are 32-bit integers in units of 2^-20 of the power of two above the largest
+// sample, each sample rounded up (2^20 + 1 at most, hence the 4,095 points).
+// It keeps the steps of large bins (32 x 32
 // cells: up to ten times the cells of a window) no coarser than those of
 // 16 x 16 bins, whose sum covers 256 cells (adjoint of 200,000 random points
 // on Kd 1024^2 against the float64 tile 1.5e-7, with the sum 2.4e-7, 16 x 16

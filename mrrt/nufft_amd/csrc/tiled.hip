@@ -29,7 +29,7 @@ void launch_tiled(bool adjoint, const TiledArgs<T, CK>& a, unsigned nsub, unsign
                           : reps ? spread_tiled_kernel<T, NDIM, CK, JMAX, FIXED, true, true>
                                  : spread_tiled_kernel<T, NDIM, CK, JMAX, FIXED, true, false>;
     if constexpr (sizeof(T) == 4 && NDIM == 2)  // finer steps in large bins
-        if (a.cmax > 0.f && (pair || !reps) && a.bg.B[0] * a.bg.B[1] > 256)
+        if (a.cmax > 0.f && (pair || !reps) && a.bg.B[0] * a.bg.B[1] > 256 && a.bg.P <= kWindowMaxP)
             spread = pair ? spread_tiled_kernel<T, NDIM, CK, JMAX, FIXED, true, false, 2, true>
                           : spread_tiled_kernel<T, NDIM, CK, JMAX, FIXED, true, false, 1, true>;
     auto interp = a.rc > 1 ? interp_tiled_kernel<T, NDIM, CK, JMAX, FIXED, true>
