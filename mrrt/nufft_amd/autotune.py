@@ -1,12 +1,11 @@
 """Autotuner for the tiled interpolation kernels.
 
 Picks the bin size, the points per subproblem and the workgroup size of the
-tiled kernels of a plan by
-timing the gather and the scatter stages on the plan's own points with HIP
-events, and caches the choice per geometry in a JSON file
+tiled kernels of a plan by timing the gather and the scatter stages on the
+plan's own points with HIP events, and caches the choice per geometry in a JSON file
 (``$MI355NUFFT_TUNE_CACHE`` or ``~/.cache/mi355nufft/autotune.json``).
-The cache key holds the library's ABI version, dimensions, image size,
-grid, kernel width, table size, precision, phasing, number of points
+The cache key holds the library's ABI version and the revision of its kernels
+(``_KERNELS``), dimensions, image size, grid, kernel width, table size, precision, phasing, number of points
 (rounded to a power of two), repetitions, frames and the scatter's
 accumulation; trajectories of the same kind and size share an entry.  An
 entry the library rejects is dropped and tuned again.
@@ -21,6 +20,11 @@ import numpy as np
 import torch
 
 from . import _lib
+
+# Revision of the timed kernels and of the rules that choose among them; raised
+# when a change moves the best choice, so that older stored choices are tuned
+# again.
+_KERNELS = 2
 
 __all__ = ["tune", "tune_fft", "candidates", "cache_path"]
 
@@ -47,8 +51,8 @@ def _key(op, nreps):
     mb = 1 << int(round(math.log2(max(op.M, 1))))
     abi = _lib.get_lib().mi355nufft_abi_version()
     fxp = int(op.plan_info()["fixed_point_scatter"])
-    return "|".join(str(v) for v in (abi, op.ndim, op.Nd, op.Kd, op.Jd, op.Ld, op.precision, op.phasing, mb, nreps,
-                                     getattr(op, "nframes", 1), fxp))
+    return "|".join(str(v) for v in (abi, _KERNELS, op.ndim, op.Nd, op.Kd, op.Jd, op.Ld, op.precision, op.phasing, mb,
+                                     nreps, getattr(op, "nframes", 1), fxp))
 
 
 def _load():
@@ -138,7 +142,9 @@ def tune(op, nreps=1, cands=None, reps=3, use_cache=True, verbose=False):
     vp = ctypes.c_void_p
     timings = {}
     best = None
-    mode = "tiled_atomic"
+    # the kernels that "auto" runs for a tile that fits (among them the scatter
+    # that owns its grid cells); other tiles are refused here
+    mode = "tiled"
     for b, p, th in cands:
         try:
             op.set_binning(b, p, mode, th)
