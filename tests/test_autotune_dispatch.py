@@ -88,3 +88,9 @@ def test_choices_of_other_kernels_are_tuned_again(op):
     json.dump({old: entry}, open(path, "w"))
     autotune.tune(op, nreps=1, cands=CANDS)
     assert len(op.timed) == 2 * first
+
+
+@pytest.mark.parametrize("bins,P", [((16, 16), 384), ((32, 16), 384), ((32, 32), 384), ((32, 16), 256), ((32, 32), 256)])
+def test_candidates_hold_the_2d_defaults(bins, P):
+    """A tuned plan is no slower than an untuned one."""
+    assert (bins, P, 256) in autotune.candidates(2)
