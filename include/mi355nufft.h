@@ -231,7 +231,12 @@ int mi355nufft_forward(mi355nufft_plan *plan, const void *x, const int64_t *xs,
  *              buffer is zero at capture (after one eager adjoint of the
  *              same nreps), and each replay leaves it zero again.  A call
  *              with a larger nreps reallocates the buffer, which ends the
- *              validity of adjoints captured before it.
+ *              validity of adjoints captured before it.  Adjoints of many 2-D
+ *              grids whose scatter writes every cell use a second plan-owned
+ *              buffer of the same size, never cleared, so a plan that runs
+ *              both kinds holds both; where the second cannot be allocated
+ *              (while capturing, or out of memory) they share the one there
+ *              is.
  */
 int mi355nufft_adjoint(mi355nufft_plan *plan, const void *y, void *x,
                        const int64_t *xs, int32_t nreps, void *grid);

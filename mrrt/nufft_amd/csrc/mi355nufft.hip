@@ -210,6 +210,40 @@ int grow_grid(mi355nufft_plan* p, int32_t nimg, void** buf, size_t* bytes) {
     return MI355NUFFT_OK;
 }
 
+// Scratch of an adjoint whose caller brings no grid.  The owner scatter, which
+// writes every cell, takes d_ogrid; every other one d_agrid, whose zeros save
+// it a clear.  Where its own is too small and cannot grow (a capture cannot
+// allocate, or memory is short) an adjoint takes the other one.  *grid is
+// d_ogrid, or stays null for d_agrid, which ends all zero either way.
+int adjoint_scratch(mi355nufft_plan* p, int32_t nimg, bool owner, void** grid) {
+    const size_t need = (size_t)nimg * (size_t)p->nk * p->cx_size();
+    size_t& mine = owner ? p->ogrid_bytes : p->agrid_bytes;
+    size_t& other = owner ? p->agrid_bytes : p->ogrid_bytes;
+    bool have = need <= mine;
+    const bool capturing = !have && stream_capturing(p);
+    if (!have && !(capturing && need <= other)) {
+        int rc = MI355NUFFT_OK;
+        auto grow = [&]() {
+            rc = owner ? grow_grid(p, nimg, &p->d_ogrid, &p->ogrid_bytes) : get_agrid(p, nimg);
+            if (rc == MI355NUFFT_ENOMEM) (void)hipGetLastError();  // not for the next launch to report
+        };
+        grow();
+        if (rc == MI355NUFFT_ENOMEM && other > 0 && need > other && !capturing) {  // room for one of them
+            HIP_TRY(hipStreamSynchronize(p->stream));
+            HIP_TRY(hipFree(owner ? p->d_agrid : p->d_ogrid));
+            (owner ? p->d_agrid : p->d_ogrid) = nullptr;
+            other = 0;
+            if (owner) p->agrid_zero = 0;
+            grow();
+        }
+        if (rc != MI355NUFFT_OK && !(rc == MI355NUFFT_ENOMEM && need <= other)) return rc;
+        have = rc == MI355NUFFT_OK;
+        if (!have) g_err.clear();
+    }
+    if (have == owner) *grid = p->d_ogrid;
+    return MI355NUFFT_OK;
+}
+
 int get_grid(mi355nufft_plan* p, int32_t nreps, void** grid) {
     if (*grid) return MI355NUFFT_OK;
     RET_IF(grow_grid(p, nreps, &p->d_grid, &p->grid_bytes));
@@ -1956,11 +1990,7 @@ int mi355nufft_adjoint(mi355nufft_plan* p, const void* y, void* x, const int64_t
     // phase: the first inverse FFT pass applies conj(phase_before) instead of
     // the scatter's flush
     const int phase = fft_phase_adjoint(p, nreps) ? 2 : 0;
-    if (!grid && !p->sp.on && use_owner(p, nreps)) {
-        // every cell is written: a grid of its own, which no pass has to clear
-        RET_IF(grow_grid(p, nimg, &p->d_ogrid, &p->ogrid_bytes));
-        grid = p->d_ogrid;
-    }
+    if (!grid) RET_IF(adjoint_scratch(p, nimg, !p->sp.on && use_owner(p, nreps), &grid));
     if (grid) {
         if (!phase) {
             RET_IF(mi355nufft_spread(p, y, grid, nreps));
@@ -1978,7 +2008,6 @@ int mi355nufft_adjoint(mi355nufft_plan* p, const void* y, void* x, const int64_t
     // clearing pass when the flag says so.  A captured adjoint ends the same
     // way on every replay: it skips the clearing pass when the grid is zero
     // at capture, and capture leaves the flag as it was.
-    RET_IF(get_agrid(p, nimg));
     const bool capturing = stream_capturing(p);
     const bool was_zero = p->agrid_zero != 0;
     const int rezero = 1;
