@@ -789,7 +789,11 @@ void default_bins(const mi355nufft_plan* p, int B[3], int& P) {
         // points per cell 44 / 42 / 44, 8 coils 132 / 115 / 108, 0.79 points
         // per cell 50 / 52 / 60; with 9,953 points on Kd 576^2 50 / 52 / 53.
         const int64_t cells = p->nframes * p->nk, bins = cells / 256;
-        if (bins >= 1024 && p->M > 16384 && 20 * p->M <= 7 * cells) {
+        // Not for the rows of a sparse matrix, which follow the bins: four
+        // repetitions of the row product on Kd 1024^2 take 289 us in 32x32 and
+        // 166 us in 16x16 order with 300,000 radial points, 356 / 229 with
+        // random ones, and in double 468 / 359.
+        if (bins >= 1024 && p->M > 16384 && 20 * p->M <= 7 * cells && !p->sparse_bins) {
             B[0] = 32;
             if (bins >= 2048) B[1] = 32;
         }

@@ -1,0 +1,26 @@
+"""Default 2-D bins of sparse k-space by mode, and transforms that equal those
+with 16x16 bins (float sums in another order and other fixed-point steps: a
+few 1e-7, 1e-14 in double)."""
+
+import numpy as np
+import pytest
+import torch
+
+from mrrt.nufft_amd import NufftBase
+from mrrt.nufft_amd import trajectories as trj
+from tests.cases import rel_l2
+
+pytestmark = pytest.mark.gpu
+
+
+def _op(Kd, m, precision="single", **kw):
+    om = np.random.default_rng(0).uniform(-np.pi, np.pi, (m, 2))
+    return NufftBase(tuple(k // 2 for k in Kd), om, Jd=6, Kd=Kd, Ld=256, precision=precision, order="C",
+                     device=torch.device("cuda", 0), **kw)
+
+
+@pytest.mark.parametrize("precision", ["single", "double"])
+@pytest.mark.parametrize("Kd", [(512, 512), (736, 720)])
+def test_sparse_matrix_rows_keep_16x16(Kd, precision):
+    A = _op(Kd, 40000, precision, mode="sparse")
+    assert A.plan_info()["bin_size"][:2] == (16, 16)
