@@ -794,8 +794,13 @@ void default_bins(const mi355nufft_plan* p, int B[3], int& P) {
         // 166 us in 16x16 order with 300,000 radial points, 356 / 229 with
         // random ones, and in double 468 / 359.
         if (bins >= 1024 && p->M > 16384 && 20 * p->M <= 7 * cells && !p->sparse_bins) {
+            // complex128: 32x32 only up to 0.1 points per cell.  Its gather
+            // stages one 22 KB tile of them at a time; 16x16 / 32x16 / 32x32,
+            // forward of 8 coils of Kd 1024^2, radial, 0.08 points per cell 202
+            // / 184 / 201 us, 0.12 206 / 189 / 209, 0.34 216 / 209 / 270; the
+            // adjoint 334 / 282 / 253, 351 / 299 / 272, 420 / 382 / 444.
             B[0] = 32;
-            if (bins >= 2048) B[1] = 32;
+            if (bins >= 2048 && (p->precision == 0 || 10 * p->M <= cells)) B[1] = 32;
         }
     } else if (fxp_eligible(p) && !p->sparse_bins) {
         // the fixed-point scatter tile of 21^3 cells takes 74 KB of LDS:

@@ -24,3 +24,16 @@ def _op(Kd, m, precision="single", **kw):
 def test_sparse_matrix_rows_keep_16x16(Kd, precision):
     A = _op(Kd, 40000, precision, mode="sparse")
     assert A.plan_info()["bin_size"][:2] == (16, 16)
+
+
+@pytest.mark.parametrize("m,bins", [(52992, (32, 32)), (52993, (32, 16)), (180000, (32, 16))])  # 0.1 per cell
+@pytest.mark.parametrize("reps", [1, 5])
+def test_double_bins_by_density(m, bins, reps):
+    A = _op((736, 720), m, "double")
+    assert A.plan_info()["bin_size"][:2] == bins
+    x = torch.from_numpy(trj.complex_gaussian((reps, 368, 360), seed=1)).cuda()
+    y = torch.from_numpy(trj.complex_gaussian((reps, m), seed=2)).cuda()
+    yf, xa = A.fft(x).cpu().numpy(), A.adj(y).cpu().numpy()
+    A.set_binning((16, 16), 384)
+    assert rel_l2(yf, A.fft(x).cpu().numpy()) <= 1e-13
+    assert rel_l2(xa, A.adj(y).cpu().numpy()) <= 1e-13
