@@ -351,6 +351,7 @@ struct TiledArgs {
     int own_ok;             // scatter: every K_d is a multiple of B_d (see spread_tiled_kernel)
     float cmax;             // scatter: > 0 accumulates in fixed point; bound of |coefficient product|
     int exact;              // gather: 1 keeps the reference's roundings (no fused multiply-add)
+    int no_cache;           // scatter: no coefficient cache, also where a subproblem has one point per thread
     int heavy;              // scatter after spread_owner_kernel: only bins of more points (0: all)
     unsigned long long* flush_count;  // scatter: non-null adds the flush's global atomic lane operations
     int flush_slots;                  // power of two: workgroup b adds to flush_count[b % flush_slots]

@@ -761,11 +761,10 @@ int fft_impl(mi355nufft_plan* p, void* grid, int32_t nreps, int direction) {
 namespace mi355host {
 
 // Default bin geometry (autotuned on golden-angle radial and kooshball
-// trajectories): 2-D 16x16 with P = 384 points per subproblem, larger on large
-// sparse grids; 3-D 16^3
-// with P = 3072 when the scatter tile is fixed point and no sparse matrix is
-// set, else 16x8x8 with P = 1024; 1-D 512 with P = 512.  Requested sizes
-// override.
+// trajectories): 2-D 16x16 with P = 384 points per subproblem, larger bins (and
+// P = 256 for few points) on large sparse grids; 3-D 16^3 with P = 3072 when
+// the scatter tile is fixed point and no sparse matrix is set, else 16x8x8
+// with P = 1024; 1-D 512 with P = 512.  Requested sizes override.
 void default_bins(const mi355nufft_plan* p, int B[3], int& P) {
     for (int d = 0; d < 3; ++d) B[d] = 1;
     if (p->ndim == 1) {
@@ -799,7 +798,15 @@ void default_bins(const mi355nufft_plan* p, int B[3], int& P) {
             // forward of 8 coils of Kd 1024^2, radial, 0.08 points per cell 202
             // / 184 / 201 us, 0.12 206 / 189 / 209, 0.34 216 / 209 / 270; the
             // adjoint 334 / 282 / 253, 351 / 299 / 272, 420 / 382 / 444.
+            // P = 256 for few points: the fullest bins of so few spokes hold
+            // up to 256 in 16x16 and more in these, a second point per thread
+            // with P = 384.  16,385 radial points on Kd 512^2, 16x16 / 32x16 with
+            // 384 / with 256: J = 7 gather 9.5 / 14.2 / 9.6 us, scatter 14.3 /
+            // 19.7 / 14.9, J = 6 forward 16.8 / 17.6 / 16.7, adjoint 20.1 / 22.1 /
+            // 21.1, gradient of 8 coils 25.5 / 40.2 / 28.4; 26,000 points, 384 /
+            // 256: forward 17.7 / 16.9, adjoint 22.7 / 21.6.
             B[0] = 32;
+            if (p->M <= 32768) P = 256;
             if (bins >= 2048 && (p->precision == 0 || 10 * p->M <= cells)) B[1] = 32;
         }
     } else if (fxp_eligible(p) && !p->sparse_bins) {

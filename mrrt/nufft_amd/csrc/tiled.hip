@@ -17,7 +17,7 @@ void launch_tiled(bool adjoint, const TiledArgs<T, CK>& a, unsigned nsub, unsign
     // tile, the sample read by the scale's sum): only when a subproblem fits
     // one point per thread (the cache costs registers even when unused:
     // 135 VGPRs against 110 for the 2-D J = 6 fixed-point scatter)
-    const bool reps = (a.ia.nreps > 1 || a.cmax > 0.f) && a.bg.P <= (int)threads;
+    const bool reps = (a.ia.nreps > 1 || a.cmax > 0.f) && a.bg.P <= (int)threads && !a.no_cache;
     // a.rc == 2 for the scatter: two repetitions' tiles per pass
     const bool pair = adjoint && a.rc == 2;
     auto spread = pair ? spread_tiled_kernel<T, NDIM, CK, JMAX, FIXED, false, false, 2>
@@ -135,8 +135,12 @@ int run_tiled(mi355nufft_plan* p, bool adjoint, const void* samples_in, void* sa
     rc = rc < nreps ? rc : nreps;
     a.rc = rc > 1 ? rc : 1;
     // the scatter takes two repetitions per pass when both tiles fit the
-    // chunk budget and its points would not fit the coefficient cache
-    if (adjoint && nreps >= 2 && kScatterPairs && 2 * one <= chunk_lds && p->bg.P > p->bg_threads) a.rc = 2;
+    // chunk budget and its points would not fit the coefficient cache, which
+    // the default points per subproblem of large bins leave out (its scale is
+    // the coarser one)
+    a.no_cache = p->ndim == 2 && p->P_req == 0 && p->bg.B[0] * p->bg.B[1] > 256;
+    if (adjoint && nreps >= 2 && kScatterPairs && 2 * one <= chunk_lds && (p->bg.P > p->bg_threads || a.no_cache))
+        a.rc = 2;
     const size_t lds = one * (size_t)a.rc;
     const int jm = jmax_of(p->ndim, J);
     const int jf = fixed_j(p->ndim, J);

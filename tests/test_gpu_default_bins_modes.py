@@ -37,3 +37,24 @@ def test_double_bins_by_density(m, bins, reps):
     A.set_binning((16, 16), 384)
     assert rel_l2(yf, A.fft(x).cpu().numpy()) <= 1e-13
     assert rel_l2(xa, A.adj(y).cpu().numpy()) <= 1e-13
+
+
+@pytest.mark.parametrize("m,P", [(16385, 256), (32768, 256), (32769, 384)])
+@pytest.mark.parametrize("precision,tol", [("single", 2e-6), ("double", 1e-13)])
+@pytest.mark.parametrize("J", [5, 7])
+def test_few_points_have_one_per_thread(m, P, precision, tol, J):
+    """Radial spokes, whose centre bins hold several subproblems, with one
+    image and a pair and a half, against 16x16 bins."""
+    om = trj.golden_angle_2d(-(-m // 256), 256)[:m]
+    A = NufftBase((256, 256), om, Jd=J, Kd=(512, 512), Ld=256, precision=precision, order="C",
+                  device=torch.device("cuda", 0))
+    info = A.plan_info()
+    assert info["bin_size"][:2] == (32, 16) and info["max_points"] == P
+    for reps in (1, 3):
+        x = torch.from_numpy(trj.complex_gaussian((reps, 256, 256), seed=1)).cuda().to(A._tcdt)
+        y = torch.from_numpy(trj.complex_gaussian((reps, m), seed=2)).cuda().to(A._tcdt)
+        A.set_binning()
+        yf, xa = A.fft(x).cpu().numpy(), A.adj(y).cpu().numpy()
+        A.set_binning((16, 16), 384)
+        assert rel_l2(yf, A.fft(x).cpu().numpy()) <= tol
+        assert rel_l2(xa, A.adj(y).cpu().numpy()) <= tol
