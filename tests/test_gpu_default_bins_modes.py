@@ -58,3 +58,20 @@ def test_few_points_have_one_per_thread(m, P, precision, tol, J):
         A.set_binning((16, 16), 384)
         assert rel_l2(yf, A.fft(x).cpu().numpy()) <= tol
         assert rel_l2(xa, A.adj(y).cpu().numpy()) <= tol
+
+
+@pytest.mark.parametrize("precision", ["single", "double"])
+@pytest.mark.parametrize("Kd,m", [((512, 512), 17000), ((512, 512), 90000), ((736, 720), 40000), ((736, 720), 180000),
+                                  ((34, 20000), 100000)])
+def test_two_phase_slots_take_no_more_than_with_16x16(Kd, m, precision):
+    """Slots beyond the budget end the reproducible scatter."""
+    A = _op(Kd, m, precision)
+
+    def slot_cells():
+        info = A.plan_info()
+        assert info["two_phase"]
+        return info["subproblem_slots"] * info["tile"]
+    A.set_binning(method="tiled_two_phase")
+    default = slot_cells()
+    A.set_binning((16, 16), 384, "tiled_two_phase")
+    assert default <= slot_cells()
