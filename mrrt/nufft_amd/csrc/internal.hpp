@@ -165,6 +165,7 @@ struct mi355nufft_plan {
     int* d_bin_i = nullptr;   // one allocation: bin_of, rank, perm (3*M_cap)
     int* d_bin_b = nullptr;   // counts, bin_start, bin_sub, bank-key counts ((3 + kBanks) * nbins_cap)
     int* d_sub = nullptr;     // sub_bin, sub_start, sub_end (3*sub_cap) + n_sub, max_count
+    int* d_max_count = nullptr;  // max_count elsewhere (raw workspaces: beside the gate word)
     void* d_tms = nullptr;    // tm in sorted order (ndim * M_cap real)
     void* d_phs = nullptr;    // per-sample phase in sorted order (M_cap complex)
     int64_t sorted_cap = 0;
@@ -247,7 +248,7 @@ inline BinState bin_state(const mi355nufft_plan* p) {
     bs.sub_start = p->d_sub + sc;
     bs.sub_end = p->d_sub + 2 * sc;
     bs.n_sub = p->d_sub + 3 * sc;
-    bs.max_count = bs.n_sub + 1;
+    bs.max_count = p->d_max_count ? p->d_max_count : bs.n_sub + 1;
     bs.frame_off = p->nframes > 1 ? p->d_frame_off : nullptr;
     bs.nframes = p->nframes;
     return bs;

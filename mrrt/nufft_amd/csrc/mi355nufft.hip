@@ -1153,7 +1153,8 @@ struct RawKey {
     }
 };
 
-// Byte offsets of one workspace: gate word, copy of tm, bin arrays
+// Byte offsets of one workspace: gate word (and, after it, the fullest bin's
+// count), copy of tm, bin arrays
 // (bin_of, rank, perm), per-bin arrays, subproblem table, sorted tm.
 struct RawLayout {
     size_t gate, tm_copy, bin_i, bin_b, sub, tms, total;
@@ -1172,7 +1173,7 @@ RawLayout raw_layout(int64_t M, int ndim, size_t rs, int64_t nbins, int64_t max_
     L.bin_b = o;
     o = up(o + (size_t)(kBanks + 3) * (size_t)nbins * sizeof(int));
     L.sub = o;
-    o = up(o + (size_t)(3 * max_sub + 2) * sizeof(int));
+    o = up(o + (size_t)(3 * max_sub + 1) * sizeof(int));
     L.tms = o;
     o = up(o + (size_t)ndim * (size_t)M * rs);
     L.total = o;
@@ -1246,6 +1247,7 @@ RawLayout raw_bind(mi355nufft_plan& q, unsigned char* base) {
     q.bin_b_cap = q.bg.nbins;
     q.d_sub = reinterpret_cast<int*>(base + L.sub);
     q.bin_s_cap = max_subproblems(&q);
+    q.d_max_count = reinterpret_cast<int*>(base + L.gate) + 1;
     q.d_tms = base + L.tms;
     q.d_phs = nullptr;
     q.binned = 1;
