@@ -40,9 +40,21 @@ TRAFFIC_BYTES = {"spread": 18007664, "interp": 12857829}
 # scatter tile; profiles/nufft3d_128_c64_hbm_traffic.md) and the 24-frame x
 # 32-coil batch (profiles/nufft2d_256_c64_frames_kernel_stats_and_traffic.md).
 TRAFFIC_BYTES_C3 = {"interp": 369.2e6, "spread": 516.4e6}
-# 64x32 bins, 1,024 points per subproblem; the scatter is spread_owner_kernel
-# and, for the dense bins, spread_tiled_kernel
-TRAFFIC_BYTES_C4 = {"interp": 2405.4e6, "spread": 2615.4e6}
+# (bin size, points per subproblem, threads) -> bytes; the scatter is
+# spread_owner_kernel and, for the dense bins, spread_tiled_kernel
+TRAFFIC_BYTES_C4 = {((64, 32), 1024, 256): {"interp": 2405.4e6, "spread": 2615.4e6}}
+
+
+def c4_traffic(info, algorithmic, gather_ms, scatter_ms):
+    """Measured HBM bytes of the batch's gather and scatter over the
+    algorithmic ones and per second, where they were counted with the bins of
+    ``info`` (plan_info); else None for both."""
+    t = TRAFFIC_BYTES_C4.get((tuple(info["bin_size"][:2]), info["max_points"], info["threads"]))
+    if t is None:
+        return {"c4_traffic_over_algorithmic": None, "c4_hbm_GBps_measured_traffic": None}
+    ms = {"interp": gather_ms, "spread": scatter_ms}
+    return {"c4_traffic_over_algorithmic": {k: round(v / algorithmic, 2) for k, v in t.items()},
+            "c4_hbm_GBps_measured_traffic": {k: round(v / (ms[k] * 1e-3) / 1e9, 1) for k, v in t.items()}}
 
 
 def parse():
@@ -303,9 +315,7 @@ def run_c4(steps=3, autotune=True, binning=None, loop=True):
             "c4_scatter_flush_atomics_per_launch": int(at4["per_launch"]),
             "c4_gather_GBps": round(b_bytes / (g_ms * 1e-3) / 1e9, 1),
             "c4_scatter_GBps": round(b_bytes / (s_ms * 1e-3) / 1e9, 1),
-            "c4_traffic_over_algorithmic": {k: round(v / b_bytes, 2) for k, v in TRAFFIC_BYTES_C4.items()},
-            "c4_hbm_GBps_measured_traffic": {"interp": round(TRAFFIC_BYTES_C4["interp"] / (g_ms * 1e-3) / 1e9, 1),
-                                             "spread": round(TRAFFIC_BYTES_C4["spread"] / (s_ms * 1e-3) / 1e9, 1)}}
+            **c4_traffic(B.op.plan_info(), b_bytes, g_ms, s_ms)}
 
 
 def run_c5(steps=5):
