@@ -35,7 +35,6 @@ namespace mi355 {
 
 constexpr int kFftMinK = 16;
 constexpr int kFftMaxK = 2048;
-constexpr int kFftMaxThreads = 1024;
 constexpr int kFftMaxPasses = 6;
 constexpr int kFftMaxRadix = 10;  // of the mixed lengths
 
@@ -75,10 +74,11 @@ struct FftAxis {
 // spreads the strided writes of the passes over the banks.
 __host__ __device__ constexpr int fft_pad(int t) { return t + (t >> 3); }
 
-// Stride of lpw lines in LDS (the mixed lengths have no unused slots: their
-// first radix is odd where one is, so their first writes have an odd stride): 32 / lpw (16 / lpw for complex128) modulo
-// 32 (16) slots, so that the lanes of lpw neighbouring lines and
-// consecutive points fall on different banks.
+// Stride of lpw lines in LDS: 32 / lpw (16 / lpw for complex128) modulo 32 (16)
+// slots, so that the lanes of lpw neighbouring lines and consecutive points
+// fall on different banks.  Lines of the mixed lengths have no unused slots:
+// their first radix is odd where one is, so their first writes have an odd
+// stride.
 __host__ __device__ constexpr int fft_line_stride(int K, int lpw, int cxs) {
     const int unit = 256 / cxs;
     const int want = lpw < unit ? unit / lpw : 1;
