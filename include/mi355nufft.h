@@ -127,8 +127,7 @@ int64_t mi355nufft_num_points(const mi355nufft_plan *plan);
  *   bin_size    ndim bin sizes in grid points (NULL or 0 entries: defaults
  *               2-D 16x16, or 32x16 / 32x32 with more than 16,384 points, at
  *               most 0.35 per grid point, from 1,024 / 2,048 bins of 16x16 on
- *               (32x32 for complex128 up to 0.1 per grid point; not with a
- *               sparse matrix set);
+ *               (not with a sparse matrix set);
  *               3-D 16x16x16 for complex64 with the fixed-point
  *               scatter tile and no sparse matrix set, else 16x8x8; 1-D
  *               512; the scatter tile, 8 bytes

@@ -793,11 +793,6 @@ void default_bins(const mi355nufft_plan* p, int B[3], int& P) {
         // 166 us in 16x16 order with 300,000 radial points, 356 / 229 with
         // random ones, and in double 468 / 359.
         if (bins >= 1024 && p->M > 16384 && 20 * p->M <= 7 * cells && !p->sparse_bins) {
-            // complex128: 32x32 only up to 0.1 points per cell.  Its gather
-            // stages one 22 KB tile of them at a time; 16x16 / 32x16 / 32x32,
-            // forward of 8 coils of Kd 1024^2, radial, 0.08 points per cell 202
-            // / 184 / 201 us, 0.12 206 / 189 / 209, 0.34 216 / 209 / 270; the
-            // adjoint 334 / 282 / 253, 351 / 299 / 272, 420 / 382 / 444.
             // P = 256 for few points: the fullest bins of so few spokes hold
             // up to 256 in 16x16 and more in these, a second point per thread
             // with P = 384.  16,385 radial points on Kd 512^2, 16x16 / 32x16 with
@@ -809,7 +804,7 @@ void default_bins(const mi355nufft_plan* p, int B[3], int& P) {
             // repetition, and adds atomically, no longer reproducibly, where
             // they would take more than 8 GB: larger bins only where their
             // slots take no more than those of 16x16.
-            const int b1 = bins >= 2048 && (p->precision == 0 || 10 * p->M <= cells) ? 32 : 16;
+            const int b1 = bins >= 2048 ? 32 : 16;
             const int pl = p->M <= 32768 ? 256 : 384;
             auto slots = [&](int64_t B0, int64_t B1, int64_t pts) {
                 B0 = B0 < p->K[0] ? B0 : p->K[0];

@@ -98,6 +98,18 @@ int run_owner(mi355nufft_plan* p, const TiledArgs<float, CK>& a, hipEvent_t ev0)
     return launch_owner<CK, 8, false>(p, a, ev0);
 }
 
+// Repetitions staged together by the gather and the gradient where only one
+// tile fits the chunk: two for the compiled tap loops (complex128 tiles of
+// 32x32 bins, 22 KB).  8 coils on Kd 1024^2, J = 6, one / two tiles, 0.33 points
+// per cell gather 165 / 108 us, gradient 217 / 176; forward of 4 frames x 32
+// coils on Kd 512^2 977 / 749.  Not for two or three repetitions, whose single
+// tiles run side by side (20,000 points on Kd 600^2, two, gather 13.4 / 15.1), nor
+// for the generic loops (J = 7, eight: 40.7 / 46.1).
+inline int pair_rather_than_one(const mi355nufft_plan* p, int rc, size_t one, size_t chunk, int32_t nreps) {
+    const int32_t J[3] = {p->J[0], p->J[1], p->J[2]};
+    return rc == 1 && nreps >= 4 && fixed_j(p->ndim, J) && 2 * one <= (chunk * 13) / 10 ? 2 : rc;
+}
+
 template <typename T, bool CK>
 int run_tiled(mi355nufft_plan* p, bool adjoint, const void* samples_in, void* samples_out, const void* grid_in,
               void* grid_out, int32_t nreps) {
@@ -131,6 +143,7 @@ int run_tiled(mi355nufft_plan* p, bool adjoint, const void* samples_in, void* sa
     const size_t one = adjoint ? tile_bytes(p) : gather_tile_bytes(p);
     const size_t chunk_lds = p->lds_limit < kRepChunkLds ? p->lds_limit : kRepChunkLds;
     int rc = adjoint ? 1 : (int)(chunk_lds / one);
+    if (!adjoint) rc = pair_rather_than_one(p, rc, one, chunk_lds, nreps);
     rc = rc < kMaxRepChunk ? rc : kMaxRepChunk;
     rc = rc < nreps ? rc : nreps;
     a.rc = rc > 1 ? rc : 1;
@@ -220,6 +233,7 @@ int run_grad(mi355nufft_plan* p, const void* grid, const void* w, void* grad, in
         const size_t chunk = p->lds_limit < kRepChunkLds ? p->lds_limit : kRepChunkLds;
         const size_t one = gather_tile_bytes(p);
         int rc = (int)((nreps <= kMaxRepChunk && nreps * one <= (chunk * 13) / 10 ? nreps * one : chunk) / one);
+        rc = pair_rather_than_one(p, rc, one, chunk, nreps);
         rc = rc < kMaxRepChunk ? rc : kMaxRepChunk;
         rc = rc < nreps ? rc : nreps;
         a.rc = rc > 1 ? rc : 1;

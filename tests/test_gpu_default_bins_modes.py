@@ -8,6 +8,7 @@ import torch
 
 from mrrt.nufft_amd import NufftBase
 from mrrt.nufft_amd import trajectories as trj
+from mrrt.nufft_amd.autograd import nufft
 from tests.cases import rel_l2
 
 pytestmark = pytest.mark.gpu
@@ -26,17 +27,23 @@ def test_sparse_matrix_rows_keep_16x16(Kd, precision):
     assert A.plan_info()["bin_size"][:2] == (16, 16)
 
 
-@pytest.mark.parametrize("m,bins", [(52992, (32, 32)), (52993, (32, 16)), (180000, (32, 16))])  # 0.1 per cell
-@pytest.mark.parametrize("reps", [1, 5])
-def test_double_bins_by_density(m, bins, reps):
-    A = _op((736, 720), m, "double")
-    assert A.plan_info()["bin_size"][:2] == bins
+@pytest.mark.parametrize("J", [4, 5, 6, 7])  # two 32x32 tiles at a time for J = 4 to 6 and four coils or more
+@pytest.mark.parametrize("reps", [3, 4, 5])
+def test_double_gather_and_gradient_of_several_coils(J, reps):
+    om = torch.from_numpy(np.random.default_rng(0).uniform(-np.pi, np.pi, (60000, 2))).cuda()
+    A = NufftBase((368, 360), om, Jd=J, Kd=(736, 720), Ld=256, precision="double", order="C", device=om.device)
     x = torch.from_numpy(trj.complex_gaussian((reps, 368, 360), seed=1)).cuda()
-    y = torch.from_numpy(trj.complex_gaussian((reps, m), seed=2)).cuda()
-    yf, xa = A.fft(x).cpu().numpy(), A.adj(y).cpu().numpy()
-    A.set_binning((16, 16), 384)
-    assert rel_l2(yf, A.fft(x).cpu().numpy()) <= 1e-13
-    assert rel_l2(xa, A.adj(y).cpu().numpy()) <= 1e-13
+    w = torch.from_numpy(trj.complex_gaussian((reps, 60000), seed=2)).cuda()
+    got = []
+    for bins in ((32, 32), (16, 16)):
+        if bins == (16, 16):
+            A.set_binning(bins, 384)
+        o = om.clone().requires_grad_(True)
+        y = nufft(A, x, o)
+        assert A.plan_info()["bin_size"][:2] == bins
+        got.append((y.detach().cpu().numpy(), torch.autograd.grad(y, (o,), w)[0].cpu().numpy()))
+    for u, v in zip(*got):
+        assert rel_l2(u, v) <= 1e-13
 
 
 @pytest.mark.parametrize("m,P", [(16385, 256), (32768, 256), (32769, 384)])
