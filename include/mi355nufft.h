@@ -141,7 +141,8 @@ int64_t mi355nufft_num_points(const mi355nufft_plan *plan);
  *               3 tiled with the scatter flushed by global atomics,
  *               4 tiled with the two-phase scatter (tile slots + one
  *               reduction per grid point in a fixed order: bit-reproducible
- *               adjoints; needs the slots to fit 8 GiB and bins not smaller
+ *               adjoints; needs the slots to fit 8 GiB (with the default 2-D
+ *               bins, those of 16x16 bins) and bins not smaller
  *               than the kernel overlap allows)
  * Re-sorts the current points if any.
  */

@@ -800,23 +800,9 @@ void default_bins(const mi355nufft_plan* p, int B[3], int& P) {
             // 19.7 / 14.9, J = 6 forward 16.8 / 17.6 / 16.7, adjoint 20.1 / 22.1 /
             // 21.1, gradient of 8 coils 25.5 / 40.2 / 28.4; 26,000 points, 384 /
             // 256: forward 17.7 / 16.9, adjoint 22.7 / 21.6.
-            // The two-phase scatter (method 4) keeps a slot per subproblem and
-            // repetition, and adds atomically, no longer reproducibly, where
-            // they would take more than 8 GB: larger bins only where their
-            // slots take no more than those of 16x16.
-            const int b1 = bins >= 2048 ? 32 : 16;
-            const int pl = p->M <= 32768 ? 256 : 384;
-            auto slots = [&](int64_t B0, int64_t B1, int64_t pts) {
-                B0 = B0 < p->K[0] ? B0 : p->K[0];
-                B1 = B1 < p->K[1] ? B1 : p->K[1];
-                const int64_t n = p->nframes * ((p->K[0] + B0 - 1) / B0) * ((p->K[1] + B1 - 1) / B1);
-                return (n + (p->M + pts - 1) / pts) * (B0 + p->J[0] - 1) * (B1 + p->J[1] - 1);
-            };
-            if (p->method != 4 || slots(32, b1, pl) <= slots(16, 16, 384)) {
-                B[0] = 32;
-                B[1] = b1;
-                P = pl;
-            }
+            B[0] = 32;
+            if (bins >= 2048) B[1] = 32;
+            if (p->M <= 32768) P = 256;
         }
     } else if (fxp_eligible(p) && !p->sparse_bins) {
         // the fixed-point scatter tile of 21^3 cells takes 74 KB of LDS:
@@ -964,8 +950,20 @@ size_t two_phase_bytes(const mi355nufft_plan* p, int32_t nreps) {
     return (size_t)max_subproblems(p) * (size_t)nreps * (size_t)p->bg.tile * p->cx_size();
 }
 
+// Slots beyond the budget are flushed with atomics instead, no longer
+// reproducibly.  The larger default bins of sparse 2-D grids take up to 1.25 times
+// the slots of 16x16 bins (0.35 points per cell); the budget counts the
+// smaller of the two, so that they do not move the line.
 bool use_two_phase(const mi355nufft_plan* p, int32_t nreps) {
-    return p->method == 4 && p->reduce_ok && two_phase_bytes(p, nreps) <= kTileSlotBudget;
+    if (p->method != 4 || !p->reduce_ok) return false;
+    size_t bytes = two_phase_bytes(p, nreps);
+    if (p->ndim == 2 && !p->bin_req[0] && !p->bin_req[1] && !p->P_req) {
+        const int64_t B0 = p->K[0] < 16 ? p->K[0] : 16, B1 = p->K[1] < 16 ? p->K[1] : 16;
+        const int64_t subs = p->nframes * ((p->K[0] + B0 - 1) / B0) * ((p->K[1] + B1 - 1) / B1) + (p->M + 383) / 384;
+        const size_t small = (size_t)(subs * (B0 + p->J[0] - 1) * (B1 + p->J[1] - 1)) * (size_t)nreps * p->cx_size();
+        bytes = bytes < small ? bytes : small;
+    }
+    return bytes <= kTileSlotBudget;
 }
 
 template <typename T>
