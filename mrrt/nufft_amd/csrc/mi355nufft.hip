@@ -397,6 +397,13 @@ bool pow2_fft_sizes_ok(int ndim, const int64_t* Kd, size_t cx_size) {
 // transform in one launch), 120 x 120 22.4 / 34.5 us, 360 x 300 26.8 /
 // 38.5 us, eight times 640 x 640 72.5 / 122.7 us, 24^3 29.9 / 34.3 us,
 // 192 x 180 x 120 134 / 179 us; one axis of 1000 15.0 / 12.9 us.
+// A single image loses by up to 5 us where rocFFT has a fast kernel for the
+// length, which no rule on sizes tells apart: 112 x 112 21.9 / 19.5, 160 x 160
+// 23.0 / 20.9, 240 x 240 24.0 / 19.0, 343 x 343 25.7 / 22.1, 1000 x 100 26.8 / 20.7
+// (four images 21.6 / 20.0, 22.6 / 22.0, 24.0 / 23.3, 28.4 / 37.2, 28.5 / 30.5).
+// The fused passes are taken there too: a first call makes no rocFFT plan (0.13
+// instead of 5 ms), and mi355nufft_set_fft chooses rocFFT where only the repeated
+// call counts.
 constexpr int64_t kFftMixedMin = 96 * 96;
 bool fused_fft_sizes_ok(int ndim, const int64_t* Kd, size_t cx_size) {
     if (pow2_fft_sizes_ok(ndim, Kd, cx_size)) return true;
