@@ -794,6 +794,10 @@ void default_bins(const mi355nufft_plan* p, int B[3], int& P) {
         // 286 / 247 / 219; Kd 512^2 (1,024 bins of 16x16), 0.25 random
         // points per cell 44 / 42 / 44, 8 coils 132 / 115 / 108, 0.79 points
         // per cell 50 / 52 / 60; with 9,953 points on Kd 576^2 50 / 52 / 53.
+        // The line at 1,024 bins is that of one image (20,000 radial points, Kd
+        // 400^2 46.7 / 49.4 / 47.8, 480^2 48.0 / 49.5 / 49.6, 504^2 52.4 / 49.5 /
+        // 49.7); eight coils gain on both sides of it (480^2 117 / 111 / 101,
+        // 504^2 132 / 115 / 108), but the points are sorted without knowing them.
         const int64_t cells = p->nframes * p->nk, bins = cells / 256;
         // Not for the rows of a sparse matrix, which follow the bins: four
         // repetitions of the row product on Kd 1024^2 take 289 us in 32x32 and
